@@ -586,7 +586,9 @@ __device__ __forceinline__ int rec_tail_cmp(wave_tile<T, C>& c, const u32* key, 
 template <u32 T, bool Validate, bool C>
 __device__ __forceinline__ void scan_read(wave_tile<T, C>& c, u32 idx, gpu_node& n) {
   for (u32 spin = 0; spin < (1u << 20); spin++) {
-    if (c.template read_node<Validate>(idx, n)) return;
+    if (c.template read_node<Validate>(idx, n) &&
+        (!Validate || !hdr_border(c.header(n)) || still_current<Validate>(c, idx, c.header(n))))
+      return;
     if (c.failed()) return;
     __builtin_amdgcn_s_sleep(1);
   }

@@ -14,8 +14,8 @@
 // outstanding memory operation of the wave (s_waitcnt vmcnt(0)) behind a compiler
 // barrier.  No C++ acquire/release fences are used on these paths: on gfx950 they are
 // whole-L2 write-back/invalidate operations.
-//   * Validated read: the whole line (header included) in one relaxed atomic load; a
-//     locked header fails; order(); the header is loaded again and must be unchanged.
+//   * Validated read: the header (a locked one fails); order(); the whole line; then, after
+//     order(), the header once more, unchanged -- or a lock from that header, below.
 //   * Lock: compare-and-swap of the unlocked header seen by a validated read (relaxed),
 //     then order() before any store to the node.
 //   * Write + unlock: relaxed atomic stores of the node, order() (the stores are
@@ -185,13 +185,15 @@ struct wave_tile {
       const u32 tag = ballot(slot < kTagSlots && (slot_hi(n.s) >> 31) != 0) & 0xFFu;
       if (!hdr_border(h) && !hdr_locked(h) && tag == hdr_tag(h)) return true;
     }
-    // seqlock read: the whole line (header included) in one load, then the header again
-    n.s = dev::coherent_load(p);
-    const u32 h = bcast(slot_lo(n.s), kMetaSlot);
+    // seqlock read: the header, then the line.  The header has to come first: the pieces of
+    // a line load need not be read together, so a line whose entries are older than its
+    // header looks valid to a check that follows (a writer's whole update fits between).
+    const u32 h = dev::coherent_load(hdr_ptr(idx));
     if (hdr_locked(h)) return false;
     dev::order();
-    const u32 h2 = dev::coherent_load(hdr_ptr(idx));
-    return h2 == h;
+    n.s = dev::coherent_load(p);
+    if (bcast(slot_lo(n.s), kMetaSlot) != h) return false;
+    return hdr_border(h) || still_current<true>(*this, idx, h);
   }
   __device__ __forceinline__ void read_node_locked(u32 idx, node_t& n) {
     n.s = dev::coherent_load(slab(idx) + slot);

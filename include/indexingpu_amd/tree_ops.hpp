@@ -243,6 +243,16 @@ IGPU_HD void op_next_layer(S& st, u32 root) {
   st.phase = ph_descend;
 }
 
+// The second half of a validated read of a border node: it still has the header its image
+// was read under, so the image is whole.  Made before anything but a lock attempt from that
+// header, which makes the same check, is based on the image's entries.
+template <bool Validate, class C>
+IGPU_HD bool still_current(C& c, u32 idx, u32 h) {
+  if (!Validate) return true;
+  c.fence_release();  // the image has been read
+  return c.peek_header(idx) == h;
+}
+
 // Builds the entry that stores `rq`'s value at a key that ends at this slice.
 template <class C>
 IGPU_HD bool make_value_entry(C& c, const request& rq, u32& ks, u32& val) {
@@ -447,11 +457,17 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
         return true;
       }
       if (q > c.high(n) && c.sibling(n) != kInvalid) {
+        if (!still_current<Validate>(c, st.node, h)) return false;
         st.node = c.sibling(n);
         return true;
       }
       u32 ks = 0, val = 0;
       const int pos = c.lookup(n, q, more, ks, val);
+      // every outcome but a lock attempt rests on the entries read: they must be whole
+      const bool lock = rq.kind != op_find && !(pos >= 0 && ks == kLink) &&
+                        !(rq.kind == op_insert && pos >= 0 && !more) &&
+                        !((rq.kind == op_erase || rq.kind == op_update) && pos < 0);
+      if (!lock && !still_current<Validate>(c, st.node, h)) return false;
       if (rq.kind == op_find) {
         if (pos < 0) {
           op_finish(st, 0);
@@ -863,6 +879,7 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
         return true;
       }
       if (q > c.high(n) && c.sibling(n) != kInvalid) {
+        if (!still_current<Validate>(c, st.node, h)) return false;
         st.node = c.sibling(n);
         return true;
       }
@@ -873,7 +890,9 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
         return true;
       }
       u32 ks = 0, val = 0;
-      if (c.lookup(n, q, true, ks, val) < 0 || ks != kLink) {
+      const int pos = c.lookup(n, q, true, ks, val);
+      if (!still_current<Validate>(c, st.node, h)) return false;
+      if (pos < 0 || ks != kLink) {
         // the path to the emptied layer is gone (not expected: only the holder of a
         // layer root's lock removes its LINK, and a layer with a LINK is not empty)
         revive_layer_root(c, st.a0);
