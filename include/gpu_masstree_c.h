@@ -193,7 +193,7 @@ int gmt_set_find_passes(gmt_index* index, uint32_t passes);
  * do not depend on it. */
 int gmt_set_record_tile(gmt_index* index, uint32_t record_tile);
 
-/* Mixed batches of at least min_requests requests (default 16384) run their finds as a
+/* Mixed batches of at least min_requests requests (default 8192) run their finds as a
  * read-only pass with the narrow two-pass kernels, then the other requests; 0 splits
  * every batch, 0xFFFFFFFF none.  The first split batch at a new largest size allocates
  * 4 bytes per request of scratch and synchronizes.  A tuning knob with no counterpart in
@@ -208,6 +208,15 @@ int gmt_set_mixed_split(gmt_index* index, uint32_t min_requests);
  * which synchronizes).  A tuning knob with no counterpart in the reference; results do
  * not depend on it. */
 int gmt_set_write_hints(gmt_index* index, uint32_t min_requests);
+
+/* Hinted write batches of at least min_requests requests (default 8192), and split mixed
+ * batches of at least twice as many, apply their writes border node by border node before
+ * the step machine runs what is left; 0xFFFFFFFF turns this off.  Uses scratch beside the
+ * hints: 4 bytes per request and a table of 512 MB at most, about 64 bytes per request of
+ * up to 4M (allocated at the first larger batch, which synchronizes; under graph capture
+ * only scratch that is there is used).  A tuning knob with no counterpart in
+ * the reference; results do not depend on it. */
+int gmt_set_write_groups(gmt_index* index, uint32_t min_requests);
 
 /* Allocates now the scratch that two-pass finds and split mixed batches use (4 bytes per
  * request) for batches of up to max_requests requests; without it the first larger

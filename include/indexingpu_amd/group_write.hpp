@@ -1,0 +1,607 @@
+// Grouped writes: the write requests of a batch applied border node by border node.
+//
+// The step machine (tree_ops.hpp) runs one write per tile: lock the border node by
+// compare-and-swap, edit, publish.  The four tiles of a wave are at different steps, so a
+// wave pays the memory round trips of each in turn (about 55 us a write), and every write
+// of a node locks and rewrites it by itself.  Large batches instead go through
+//   1. the hint descent (narrow_find.hpp): the border node of every write;
+//   2. group_build_kernel: the writes of one border node join one slot of a hash table
+//      over node indices;
+//   3. group_write_kernel: one 16-lane tile takes one border node and applies up to 16 of
+//      its writes at once, lane r holding request r.  No other writer touches the node (all
+//      of its writes are in its slot, launches that write are ordered on one stream), so
+//      there is no lock to win and nothing to validate: the tiles of a wave go through one
+//      straight sequence together and share each memory round trip.  A node that overflows
+//      is split in two; its parent is left to
+//   4. batch_kernel, which runs what is left: the link of each new right node into its
+//      parent (op_link) and the requests that step 3 does not do -- further trie layers,
+//      push-downs, a second request for one entry, the erase that empties a node, nodes with
+//      more requests than a tile takes.
+// Readers that run beside the batch (find<concurrent>, scan<concurrent> on other streams)
+// see what they see of the step machine: the header is locked before the first store to a
+// node, every store is coherent and complete before the unlocked header is stored.
+//
+// Measured on MI355X (16M keys of 2..8 slices, 2-slice values), the launches that write: 4M
+// inserts 5.0 -> 1.5 ms, 4M erases 3.4 -> 1.0 ms, 1M updates of 8-slice values on 4M keys
+// 1.03 -> 0.46 ms, the 105K writes of a 1M mixed batch on 64M keys 0.27 -> 0.11 ms.
+#pragma once
+#include "kernels.hpp"
+
+namespace indexingpu_amd {
+
+// Scratch of a launch: a hash table over border nodes.  heads[s] = (node + 1, requests that
+// joined), 0 where no node has slot s (all of it between launches); body[s * room + r] is
+// the r-th request to join: launch position, slice in the node's layer, tail length | value
+// length << 16, kind | layer << 8.  `status` has a word per launch position
+// (batch_args::status).
+struct group_view {
+  u64* heads;
+  uint4* body;
+  u32 slots;  // a power of two, at least 64
+  u32 room;   // requests a slot holds: a power of two, at most kGroupTake
+  u32* status;
+  u32* claims;  // first of the bitmap words that group_write_kernel's waves begin with
+  u32 waves;    // those waves (0: the launch stores no records)
+  u32 words;    // bitmap words a wave takes from the claim cursor at once
+  u32 window;   // table slots a wave takes at once (4 .. 64)
+};
+constexpr u32 kGroupTake = 16;    // requests of one node that one tile applies
+constexpr u32 kGroupProbes = 32;  // table slots a request looks at
+
+__device__ __forceinline__ u64 launch_range(const batch_args& a, u64& lo) {
+  u64 hi = a.n;
+  lo = 0;
+  if (a.range) {
+    hi = min(a.range[1], a.n);
+    lo = min(a.range[0], hi);
+  }
+  return hi;
+}
+
+// Bound by the table's random lines: a load, a compare-and-swap for the first request of a
+// node, an add and the request's 16 bytes.  It reads what the groups need of each request in
+// launch order, so group_write_kernel gathers key and value rows only.  A node that more
+// than 16 lanes of one wave want is hot (a batch past the tree's right edge): its slot could
+// hold 16 of them anyway, and thousands of adds on one address would queue, so those
+// requests are left to batch_kernel.
+__global__ void __launch_bounds__(kBlockThreads) group_build_kernel(batch_args a, group_view g,
+                                                                     slab_pool_view pool) {
+  if (g.waves && blockIdx.x == 0 && threadIdx.x == 0)
+    *g.claims = dev::atomic_add(pool.cursor, g.waves * g.words);
+  const u32 num_slabs = pool.num_slabs;
+  u64 lo;
+  const u64 hi = launch_range(a, lo);
+  const u32 n = (u32)(hi - lo);
+  const u32 mask = g.slots - 1;
+  const u32 stride = gridDim.x * kBlockThreads;
+  const u32 maxK = a.max_key_length, maxV = a.max_value_length;
+  for (u32 p0 = blockIdx.x * kBlockThreads; p0 < n; p0 += stride) {
+    const u32 p = p0 + threadIdx.x;
+    u32 node = kInvalid, status = kStatusNone;
+    uint4 req = make_uint4(p, 0, 0, 0);
+    if (p < n) {
+      const u64 i = request_index(a, lo + p);
+      const u32 kind = a.types ? (u32)a.types[i] : a.kind;
+      if (kind != op_find) {
+        status = kStatusOpen;  // batch_kernel's unless a group decides it
+        const uint4 hint = *reinterpret_cast<const uint4*>(a.hints + (u64)kHintWords * p);
+        const u32 l = hint.w;
+        const u32 L = a.key_lengths ? a.key_lengths[i] : maxK;
+        const bool writes = kind != op_erase;
+        const u32 vlen = !writes ? 0u : (a.value_lengths ? a.value_lengths[i] : maxV);
+        if (hint.x < num_slabs && kind <= op_upsert && l < L && L <= maxK && vlen <= maxV &&
+            vlen <= kMaxLength && L - l - 1 <= kMaxLength &&
+            rec_num_slabs(L - l + vlen) <= kGroupTake) {  // a tile's lanes take its slabs
+          node = hint.x;
+          req.y = a.keys[i * maxK + l];
+          req.z = (L - l - 1) | (vlen << 16);
+          req.w = kind | (l << 8);
+        }
+      }
+    }
+    const u64 have = __ballot(node != kInvalid);
+    if (have) {
+      const u32 first = (u32)__builtin_amdgcn_readlane((int)node, __ffsll((unsigned long long)have) - 1);
+      if ((u32)__popcll(__ballot(node == first)) > kGroupTake && node == first) node = kInvalid;
+    }
+    if (node != kInvalid) {
+      u32 h = (node * 0x9E3779B1u) >> 7 & mask;
+      for (u32 probe = 0; probe < kGroupProbes; probe++, h = (h + 1) & mask) {
+        const u64 cur = dev::coherent_load(g.heads + h);
+        u32* head = reinterpret_cast<u32*>(g.heads + h);
+        u32 at = slot_lo(cur);
+        if (at == 0) {
+          u32 expected = 0;
+          at = __hip_atomic_compare_exchange_strong(head, &expected, node + 1, __ATOMIC_RELAXED,
+                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                   ? node + 1
+                   : expected;
+        }
+        if (at == node + 1) {
+          if (slot_hi(cur) < g.room) {
+            const u32 r = dev::atomic_add(head + 1, 1u);
+            if (r < g.room) g.body[(u64)h * g.room + r] = req;
+          }
+          break;
+        }
+      }
+    }
+    if (p < n) g.status[p] = status;
+  }
+}
+
+// Slabs of one wave (uniform over it): the free bits of a claimed bitmap word, and the words
+// the wave goes on with.  Every cursor step is an atomic on one address for all waves, which
+// take a good 10 ns each (4M inserts: 131K steps of one word are 1.6 ms), so a wave steps by
+// g.words words, and its first ones are dealt out by group_build_kernel: words
+// [*g.claims + wave * g.words, + g.words).
+struct wave_slabs {
+  u32 word = 0;
+  u32 bits = 0;
+  u32 next = 0;  // cursor values [next, next + left) are this wave's
+  u32 left = 0;
+  bool dry = false;  // a claim failed: no further ones in this launch
+};
+
+// position of the r-th set bit of m (r < popcount)
+__device__ __forceinline__ u32 nth_set_bit(u32 m, u32 r) {
+  u32 at = 0;
+#pragma unroll
+  for (u32 w = 16; w; w >>= 1) {
+    const u32 c = (u32)__popc(m & ((1u << w) - 1u));
+    if (r >= c) {
+      r -= c;
+      m >>= w;
+      at += w;
+    }
+  }
+  return at;
+}
+
+// The next bitmap word of the wave with free slabs (ws.word, ws.bits); false: none.  The
+// word at the wave's cursor is simply taken; once one was full, the wave looks at 64 words
+// at a time (the cursor regularly enters the part of the pool that the tree fills).
+__device__ __forceinline__ bool wave_claim(const slab_pool_view& v, wave_slabs& ws, u32 words) {
+  const u32 lane = threadIdx.x & 63u;
+  if (v.limits) {  // linear allocator: the active region grows on misses
+    u32 w = 0, b = 0;
+    bool ok = true;
+    if (lane == 0) ok = dev::claim_word(v, true, w, b);
+    ws.word = (u32)__builtin_amdgcn_readfirstlane((int)w);
+    ws.bits = (u32)__builtin_amdgcn_readfirstlane((int)b);
+    return __builtin_amdgcn_readfirstlane((int)ok) != 0;
+  }
+  const u32 nw = v.num_words;
+  bool look = false;
+  for (u64 seen = 0; seen <= (u64)nw + 64;) {
+    if (ws.left == 0) {
+      const u32 step = look ? 64u : words;
+      u32 c = 0;
+      if (lane == 0) c = dev::atomic_add(v.cursor, step);
+      ws.next = (u32)__builtin_amdgcn_readfirstlane((int)c);
+      ws.left = step;
+    }
+    u32 skip = 0;  // full words in front
+    if (look) {
+      const u32 x = dev::coherent_load(&v.bitmap[(ws.next + lane) % nw]);
+      const u64 open = __ballot(lane < ws.left && x != 0xFFFFFFFFu);
+      skip = open ? (u32)__ffsll((unsigned long long)open) - 1u : min(ws.left, 64u);
+    }
+    u32 bits = 0;
+    if (skip < ws.left) {
+      ws.word = (ws.next + skip) % nw;
+      if (lane == 0) bits = ~dev::atomic_or(&v.bitmap[ws.word], 0xFFFFFFFFu);
+      ws.bits = (u32)__builtin_amdgcn_readfirstlane((int)bits);
+      skip += 1;
+    }
+    ws.next += skip;
+    ws.left -= skip;
+    seen += skip;
+    if (ws.bits) return true;
+    look = true;
+  }
+  return false;
+}
+
+// A slab for every lane with `need` (kInvalid where the pool has none).  Every lane of the
+// wave calls it.
+__device__ __forceinline__ u32 wave_alloc(const slab_pool_view& v, wave_slabs& ws, u32 words,
+                                          bool need) {
+  const u32 lane = threadIdx.x & 63u;
+  u32 idx = kInvalid;
+  u64 m = __ballot(need);
+  while (m) {
+    if (ws.bits == 0 && (ws.dry || !wave_claim(v, ws, words))) {
+      ws.dry = true;
+      break;
+    }
+    const u32 have = (u32)__popc(ws.bits), wanted = (u32)__popcll(m);
+    const u32 rank = (u32)__popcll(m & ((1ull << lane) - 1ull));
+    if (need && idx == kInvalid && rank < have) idx = ws.word * 32u + nth_set_bit(ws.bits, rank);
+    if (wanted >= have) ws.bits = 0;
+    else ws.bits &= ~0u << nth_set_bit(ws.bits, wanted);
+    m = __ballot(need && idx == kInvalid);
+  }
+  return idx;
+}
+
+// LDS written by some lanes of the wave and read by others: the wave's LDS operations run
+// in order, so only the compiler has to keep theirs.
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Compares a record's tail with key[0, len), len > 0, one lane by itself: 1 equal, 0 not, 2 a
+// slab index outside the pool.  The record's first 32 bytes and the key words they are
+// compared with are loaded at once, without branches: most tails end there, after one
+// round trip (an erase of 4M keys: 1.03 ms where the length word was waited for first).
+__device__ __forceinline__ u32 lane_tail_equal(const u64* pool, u32 num_slabs, u32 rec,
+                                               const u32* key, u32 len) {
+  if (rec >= num_slabs) return 2;
+  const u32* w = reinterpret_cast<const u32*>(pool + (u64)rec * kSlots);
+  const uint4 a = *reinterpret_cast<const uint4*>(w), b = *reinterpret_cast<const uint4*>(w + 4);
+  const u32 r[7] = {a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  u32 k[7];
+#pragma unroll
+  for (u32 t = 0; t < 7; t++) k[t] = key[min(t, len - 1)];
+  u32 diff = rec_tail_len(a.x) ^ len;
+#pragma unroll
+  for (u32 t = 0; t < 7; t++) diff |= t < len ? r[t] ^ k[t] : 0u;
+  if (diff) return 0;
+  u32 d = 8;
+  for (u32 j = 7; j < len;) {
+    if (d == kRecordWordsPerSlab) {
+      const u32 nxt = w[kRecordNextWord];
+      if (nxt >= num_slabs) return 2;
+      w = reinterpret_cast<const u32*>(pool + (u64)nxt * kSlots);
+      d = 0;
+    }
+    const u32 m = min(min(len - j, kRecordWordsPerSlab - d), 8u);
+#pragma unroll
+    for (u32 t = 0; t < 8; t++) diff |= w[d + min(t, m - 1)] ^ key[j + min(t, m - 1)];
+    if (diff) return 0;
+    j += m;
+    d += m;
+  }
+  return 1;
+}
+
+// Bound by memory latency: a group goes through about five dependent round trips (table
+// slots, node and requests, records compared, words of new records, their stores complete),
+// four groups of a wave in each; the unlocked header of a group is stored in the next
+// group's first round trip.
+template <bool Stores>
+__global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv, batch_args a,
+                                                                     group_view g) {
+  enum : u32 { aFail = 0, aInsert = 1, aReplace = 2, aDelete = 3, aRest = 4 };
+  const wave_tile<16, true> c(tv.pool, tv.retire, tv.err, tv.root);
+  const u32 lane64 = threadIdx.x & 63u, slot = c.slot, tile = lane64 >> 4;
+  const u32 below_me = (1u << slot) - 1u;
+  u64 lo;
+  launch_range(a, lo);
+  const u32 num_slabs = tv.pool.num_slabs;
+  const u32 maxK = a.max_key_length, maxV = a.max_value_length;
+  const u32 cap_bits = (a.flags >> kReqBorderCapShift) & 15u;
+  const u32 cap = cap_bits ? cap_bits : kBorderCap;
+  const u32 step = gridDim.x * (kBlockThreads / 64) * g.window;
+  // after a corruption or livelock guard fired batch_kernel skips the requests
+  const u32 err = *tv.err;
+  const bool skip = __builtin_amdgcn_readfirstlane((int)(err == kErrStepLimit || err == kErrBadIndex)) != 0;
+  __shared__ u64 image[kBlockThreads / 16][32];  // a tile's new entries, in order
+  __shared__ uint8_t half_of[kBlockThreads / 64][128];  // halves of new records, a wave's list
+  const u32 tile_in_block = threadIdx.x / 16, wave_in_block = threadIdx.x / 64;
+  wave_slabs ws;
+  if (g.waves) {
+    ws.next = *g.claims + (blockIdx.x * (kBlockThreads / 64) + threadIdx.x / 64) * g.words;
+    ws.next = (u32)__builtin_amdgcn_readfirstlane((int)ws.next);
+    ws.left = g.words;
+  }
+  u32 unlock_node = kInvalid;  // the last group's node (in lane kMetaSlot), and its header
+  u32 unlock_to = 0;
+  auto unlock = [&]() {
+    dev::order();
+    if (unlock_node != kInvalid) dev::coherent_store(c.hdr_ptr(unlock_node), unlock_to);
+    unlock_node = kInvalid;
+  };
+  u32 w0 = (blockIdx.x * (kBlockThreads / 64) + threadIdx.x / 64) * g.window;
+  const bool in_window = lane64 < g.window;
+  u64 next_entry = w0 < g.slots && in_window ? g.heads[w0 + lane64] : 0ull;
+  for (; w0 < g.slots; w0 += step) {
+    const u64 entry = next_entry;
+    next_entry = w0 + step < g.slots && in_window ? g.heads[w0 + step + lane64] : 0ull;
+    u64 todo = __ballot(slot_lo(entry) != 0);
+    if (todo == 0) continue;
+    if (slot_lo(entry) != 0) g.heads[w0 + lane64] = 0;
+    if (skip) continue;
+    while (todo) {
+      // ---- each tile takes the next group of the window
+      u32 from_slot = 64;
+#pragma unroll
+      for (u32 t = 0; t < 4; t++) {
+        if (todo == 0) break;
+        if (tile == t) from_slot = (u32)__ffsll((unsigned long long)todo) - 1u;
+        todo &= todo - 1;
+      }
+      const u32 node = __shfl(slot_lo(entry), (int)(from_slot & 63u), 64) - 1u;
+      const u32 joined = __shfl(slot_hi(entry), (int)(from_slot & 63u), 64);
+      const bool live = from_slot < 64 && node < num_slabs;
+      const u32 k = live ? min(joined, g.room) : 0u;  // lane r < k holds request r
+      gpu_node nd;
+      nd.s = live ? c.slab(node)[slot] : 0ull;
+      const bool have = slot < k;
+      uint4 req = make_uint4(0, 0, 0, 0);
+      if (have) req = g.body[(u64)(w0 + from_slot) * g.room + slot];
+      unlock();  // the last group's stores are older than these loads
+      const u32 p = req.x, q = req.y, tail = req.z & 0xFFFFu, vlen = req.z >> 16;
+      const u32 kind = req.w & 0xFFu, l = c.bcast(req.w, 0) >> 8;
+      const u32 i = have ? (u32)request_index(a, lo + p) : 0u;
+      const bool more = tail != 0;
+      // ---- the node
+      const u32 h = c.header(nd), sib = c.sibling(nd), high = c.high(nd), ksb = c.ksbits(nd);
+      const bool usable = live && hdr_border(h) && !hdr_locked(h) && hdr_level(h) == 0 &&
+                          hdr_nkeys(h) <= kBorderCap;
+      const u32 nk = usable ? hdr_nkeys(h) : 0u;
+      const u32 myks = ks_get(ksb, slot & 15u);
+      const u32 slice = slot_lo(nd.s);
+      const bool cand = usable && have && !(q > high && sib != kInvalid);
+      // the lock is stored now, beside the loads that follow
+      const bool locked = c.ballot(cand) != 0;
+      if (locked && slot == kMetaSlot) dev::coherent_store(c.hdr_ptr(node), h | kLockBit);
+      u32 layer_root = 0, parent = 0;  // for the link of a split
+      if (Stores && nk + k > cap) {
+        const u32* hp = a.hints + (u64)kHintWords * c.bcast(p, 0);
+        layer_root = hp[1];
+        parent = hp[2];
+      }
+      // ---- order of entries and requests: masks over entries (0..13) and request lanes
+      u32 below = 0;           // request lane: entries below it, | requests below it << 16
+      u32 requests_under = 0;  // entry lane: requests below the entry
+      u32 match = 16;          // request lane: the entry equal to it
+      u32 by = 16;             // entry lane: the first request equal to it
+      bool dup = false;        // request lane: an earlier request has the same entry
+      for (u32 r = 0; __ballot(r < k); r++) {
+        const u32 qr = c.bcast(q, r);
+        const u32 fr = c.bcast((cand ? 1u : 0u) | (more ? 2u : 0u), r);
+        const bool mr = (fr & 2u) != 0;
+        const bool on = (fr & 1u) != 0 && r < k;
+        const bool is_entry = slot < nk;
+        const bool lt = is_entry && entry_less(slice, ks_more(myks), qr, mr);
+        const bool eq = is_entry && slice == qr && ks_more(myks) == mr;
+        const u32 ltm = c.ballot(lt), eqm = c.ballot(eq);
+        if (on) {
+          if (slot == r) {
+            below |= ltm;
+            if (eqm) match = (u32)__builtin_ctz(eqm);
+          }
+          if (is_entry && !lt && !eq) requests_under |= 1u << r;
+          if (eq && by == 16) by = r;
+          if (cand) {
+            if (slot > r && q == qr && more == mr) dup = true;
+            if (entry_less(qr, mr, q, more)) below |= 0x10000u << r;
+          }
+        }
+      }
+      // ---- what each request does
+      const u32 mval = c.bcast(slot_hi(nd.s), match & 15u);
+      const u32 mks = ks_get(ksb, match & 15u);
+      u32 act = aRest;
+      if (cand && !dup) {
+        if (match == 16) {
+          act = (kind == op_insert || kind == op_upsert) ? aInsert : aFail;
+          if (act == aInsert && more && (a.flags & kReqNoSuffix)) act = aRest;  // a layer chain
+        } else if (mks != kLink) {
+          u32 same = 1;
+          if (mks == kSuffix)
+            same = lane_tail_equal(tv.pool.pool, num_slabs, mval, a.keys + (u64)i * maxK + l + 1, tail);
+          if (same == 1) {
+            act = kind == op_insert ? aFail : (kind == op_erase ? aDelete : aReplace);
+          } else if (same == 0) {
+            // another tail: inserts push the entry one layer down
+            act = (kind == op_erase || kind == op_update) ? aFail : aRest;
+          }
+        }
+      }
+      bool surv;           // entry lane: the entry stays
+      u32 by_act;          // entry lane: what its request does
+      u32 survm, insm, T;  // entries that stay, requests that insert, entries afterwards
+      auto settle = [&]() {
+        by_act = __shfl(act, (int)(by & 15u), 16);
+        if (by == 16) by_act = aFail;
+        surv = slot < nk && by_act != aDelete;
+        survm = c.ballot(surv);
+        insm = c.ballot(act == aInsert);
+        T = (u32)(__popc(survm) + __popc(insm));
+      };
+      settle();
+      const bool root = hdr_root(h);
+      u32 want = 0, new_node = kInvalid, first_new = kInvalid, second_new = kInvalid;  // new nodes
+      u32 new_ks = kValue, new_val = kInvalid;  // what an inserted or replaced entry holds
+      if constexpr (Stores) {
+      // at most two nodes: equal slices stay together, so up to 2 cap - 1 entries
+      {
+        const u32 ns = (u32)__popc(survm);
+        const u32 room = 2 * cap - 1 > ns ? 2 * cap - 1 - ns : 0u;
+        if (T > cap && act == aInsert && (u32)__popc(insm & below_me) >= room) act = aRest;
+      }
+      settle();
+      want = (T > cap && insm) ? (root ? 2u : 1u) : 0u;
+      new_node = wave_alloc(tv.pool, ws, g.words, slot < want);
+      first_new = c.bcast(new_node, 0);
+      second_new = c.bcast(new_node, 1);
+      if (want && (first_new == kInvalid || (want == 2 && second_new == kInvalid))) {
+        if (new_node != kInvalid) dev::free_slab(tv.pool, new_node);
+        if (act == aInsert) act = aRest;
+        want = 0;
+      }
+      // ---- records of inserted and replaced values
+      const bool store = act == aInsert || act == aReplace;
+      new_ks = more ? kSuffix : (vlen == 1 ? kValue : kLongVal);
+      const u32 total = 1 + tail + vlen;
+      const u32 slabs = rec_num_slabs(total);
+      bool rec = store && new_ks != kValue;
+      if (store && !rec) new_val = a.values[(u64)i * maxV];
+      {
+        const bool one = rec && slabs == 1;
+        const u32 s0 = wave_alloc(tv.pool, ws, g.words, one);
+        if (one) new_val = s0;
+        if (one && s0 == kInvalid) {
+          act = aRest;
+          rec = false;
+        }
+      }
+      auto word = [&](u32 ii, u32 ll, u32 tl, u32 tot, u32 d) -> u32 {
+        if (d == 0) return rec_len_word(tl, tot - 1 - tl);
+        if (d >= tot) return 0;
+        return d <= tl ? a.keys[(u64)ii * maxK + ll + d] : a.values[(u64)ii * maxV + (d - 1 - tl)];
+      };
+      // Records of one slab are stored in halves of 64 bytes (the second only where it is
+      // filled), eight lanes and one coalesced store each: the halves of the wave's four
+      // groups are listed in LDS, so the wave takes eight at a time whoever they belong to.
+      {
+        const bool one = rec && slabs == 1, two = one && total > 16;
+        const u64 m1 = __ballot(one), m2 = __ballot(two);
+        const u64 lt = (1ull << lane64) - 1ull;
+        const u32 n1 = (u32)__popcll(m1), halves = n1 + (u32)__popcll(m2);
+        if (one) half_of[wave_in_block][__popcll(m1 & lt)] = (uint8_t)lane64;
+        if (two) half_of[wave_in_block][n1 + __popcll(m2 & lt)] = (uint8_t)(lane64 | 64u);
+        lds_order();
+        for (u32 s0 = 0; s0 < halves; s0 += 16) {
+          u32 x0[2], x1[2], at[2], dd[2];
+#pragma unroll
+          for (u32 j = 0; j < 2; j++) {
+            const u32 s = s0 + 8 * j + (lane64 >> 3);
+            const u32 e = s < halves ? half_of[wave_in_block][s] : 0u;
+            const int r = (int)(e & 63u);
+            const u32 ii = __shfl(i, r, 64), ll = __shfl(l, r, 64), rz = __shfl(req.z, r, 64);
+            const u32 tl = rz & 0xFFFFu, tot = 1 + tl + (rz >> 16);
+            const u32 d = (e >> 6) * 16 + 2 * (lane64 & 7u);
+            at[j] = __shfl(new_val, r, 64);
+            dd[j] = d / 2;
+            x0[j] = x1[j] = 0;
+            if (s < halves) {
+              x0[j] = word(ii, ll, tl, tot, d);
+              x1[j] = d + 1 == kRecordNextWord ? kInvalid : word(ii, ll, tl, tot, d + 1);
+            }
+          }
+#pragma unroll
+          for (u32 j = 0; j < 2; j++)
+            if (s0 + 8 * j + (lane64 >> 3) < halves)
+              dev::coherent_store(c.slab(at[j]) + dd[j], slot_make(x0[j], x1[j]));
+        }
+      }
+      // Longer records, one of each tile at a time: their slabs are neighbours where the
+      // bitmap word has that many free, one whole-line store each.
+      for (u32 m = c.ballot(rec && slabs > 1); __ballot(m != 0); m &= m - 1) {
+        const u32 r = m ? (u32)__builtin_ctz(m) : 0u;
+        const u32 ii = c.bcast(i, r), tl = c.bcast(tail, r), tot = c.bcast(total, r);
+        u32 count = m ? rec_num_slabs(tot) : 0u;
+        const u32 idx = wave_alloc(tv.pool, ws, g.words, slot < count);
+        if ((u32)__popc(c.ballot(idx != kInvalid)) < count) {  // out of slabs: left
+          if (idx != kInvalid) dev::free_slab(tv.pool, idx);
+          if (slot == r) act = aRest;
+          count = 0;
+        }
+        const u32 head = c.bcast(idx, 0);
+        if (count && slot == r) new_val = head;
+        for (u32 s = 0; __ballot(s < count); s++) {
+          const u32 at = c.bcast(idx, s & 15u), nxt = c.bcast(idx, (s + 1) & 15u);
+          if (s >= count) continue;
+          const u32 d = s * kRecordWordsPerSlab + 2 * slot;
+          const u32 x0 = word(ii, l, tl, tot, d);
+          const u32 x1 = slot < 15 ? word(ii, l, tl, tot, d + 1) : (s + 1 < count ? nxt : kInvalid);
+          dev::coherent_store(c.slab(at) + slot, slot_make(x0, x1));
+        }
+      }
+      settle();
+      }
+      // the erase that would empty the node merges it away or unlinks its layer: left
+      {
+        const u32 delm = c.ballot(act == aDelete);
+        if (T == 0 && delm && slot == (u32)__builtin_ctz(delm)) act = aRest;
+      }
+      settle();
+      const bool split = want && T > cap;
+      if (want && !split && new_node != kInvalid) dev::free_slab(tv.pool, new_node);
+      const bool changed = c.ballot(act == aInsert || act == aReplace || act == aDelete) != 0;
+      // ---- the new images, behind the lock bit
+      dev::order();  // records are complete, the header is locked
+      const u32 opos = (u32)(__popc(survm & below_me) + __popc(requests_under & insm));
+      const u32 ipos = (u32)__popc(below & (survm | insm << 16));
+      const bool ins = act == aInsert;
+      const u32 rks = __shfl(new_ks, (int)(by & 15u), 16), rval = __shfl(new_val, (int)(by & 15u), 16);
+      const u32 oks = by_act == aReplace ? rks : myks;
+      const u32 oval = by_act == aReplace ? rval : slot_hi(nd.s);
+      u64 states = (surv ? (u64)oks << (2 * opos) : 0ull) | (ins ? (u64)new_ks << (2 * ipos) : 0ull);
+#pragma unroll
+      for (int m = 1; m < 16; m <<= 1) states |= __shfl_xor(states, m, 16);
+      auto slice_at = [&](u32 x) -> u32 {
+        const u32 b0 = c.ballot(surv && opos == x), b1 = c.ballot(ins && ipos == x);
+        const u32 v0 = c.bcast(slice, b0 ? (u32)__builtin_ctz(b0) : 0u);
+        const u32 v1 = c.bcast(q, b1 ? (u32)__builtin_ctz(b1) : 0u);
+        return b0 ? v0 : v1;
+      };
+      u32 cut = (T + 1) / 2, sep = 0;
+      if (__ballot(split)) {
+        if (slice_at(cut - 1) == slice_at(cut)) cut -= 1;
+        sep = slice_at(cut - 1);
+      }
+      if (!split) cut = T;
+      const u32 left = (split && root) ? first_new : node;
+      const u32 right = root ? second_new : first_new;
+      // entries in order, staged so that each node is one store of its whole line
+      image[tile_in_block][slot] = 0;
+      image[tile_in_block][slot + 16] = 0;
+      lds_order();
+      if (surv) image[tile_in_block][opos] = slot_make(slice, oval);
+      if (ins) image[tile_in_block][ipos] = slot_make(q, new_val);
+      lds_order();
+      u64 lv = slot < cut ? image[tile_in_block][slot] : 0ull;
+      u64 rv = image[tile_in_block][(cut + slot) & 31u];  // 0 past the last entry
+      if (slot == kHighSlot)
+        lv = slot_make(split ? sep : high, (u32)(states & ((1ull << (2 * cut)) - 1ull)));
+      if (slot == kMetaSlot)
+        lv = (split && root) ? slot_make(hdr_make(cut, true, false, 0), right)
+                             : slot_make(hdr_with_nkeys(h, cut) | kLockBit, split ? right : sib);
+      if (changed) dev::coherent_store(c.slab(left) + slot, lv);
+      if (split) {
+        if (slot == kHighSlot) rv = slot_make(high, (u32)(states >> (2 * cut)));
+        if (slot == kMetaSlot) rv = slot_make(hdr_make(T - cut, true, false, 0), root ? kInvalid : sib);
+        dev::coherent_store(c.slab(right) + slot, rv);
+        if (root) {
+          // the layer root becomes the parent of the two halves, in place
+          const u32 ih = (h & ~((1u << kVersionShift) - 1u)) | kLockBit | hdr_make(2, false, true, 1);
+          u64 v = 0;
+          if (slot == 0) v = slot_make(sep, left);
+          if (slot == 1) v = slot_make(kMaxSlice, right);
+          if (slot == kMetaSlot) v = slot_make(ih, kInvalid);
+          if (slot < kTagSlots) v |= (u64)((hdr_publish_tag(ih) >> slot) & 1u) << 63;
+          dev::coherent_store(c.slab(node) + slot, v);
+        }
+      }
+      // stored once every store above is complete
+      if (locked && slot == kMetaSlot) {
+        const u32 body = (split && root) ? hdr_make(2, false, true, 1)
+                                         : (hdr_with_nkeys(h, cut) & ((1u << kVersionShift) - 1u));
+        unlock_node = node;
+        unlock_to = changed ? hdr_unlocked_next((h & ~((1u << kVersionShift) - 1u)) | body) : h;
+      }
+      // ---- outcomes
+      if (have && act != aRest) {
+        u32 status = act == aFail ? kStatusFail : kStatusDone;
+        if ((act == aReplace || act == aDelete) && ks_record(mks)) status = kStatusRecord | mval;
+        if (split && !root && ins && (insm & below_me) == 0) {
+          // the first inserting position carries the right node's link into the parent
+          *reinterpret_cast<uint4*>(a.hints + (u64)kHintWords * p) =
+              make_uint4(right, sep, layer_root, parent);
+          status = kStatusLink;
+        }
+        g.status[p] = status;
+      }
+    }
+  }
+  unlock();
+  if (ws.bits != 0 && lane64 == 0) dev::atomic_and(&tv.pool.bitmap[ws.word], ~ws.bits);
+}
+
+}  // namespace indexingpu_amd

@@ -94,8 +94,20 @@ struct batch_args {
   // kReqNoSuffix (insert / upsert with enable_suffix = false), kReqKeepEmptyLayers
   // (erase<do_remove_empty_root = false>), kReqNoMerge (erase<..., do_merge = false>)
   u32 flags;
+  // Optional statuses of the launch positions, as group_write_kernel leaves them:
+  // batch_kernel runs the requests and links that are open and passes over the others.
+  const u32* status;
 };
 constexpr u32 kHintWords = 4;
+
+// Statuses of launch positions (group_write.hpp).
+constexpr u32 kStatusOpen = 0xFFFFFFFFu;    // left to batch_kernel
+constexpr u32 kStatusLink = 0xFFFFFFFEu;    // succeeded; its hint words hold a link (op_link)
+constexpr u32 kStatusDone = 0xFFFFFFFDu;    // succeeded
+constexpr u32 kStatusFail = 0xFFFFFFFCu;    // failed (stored already, or absent)
+constexpr u32 kStatusNone = 0xFFFFFFFBu;    // not a write
+constexpr u32 kStatusRecord = 0x80000000u;  // succeeded; bits 0-30: the record it replaced
+__device__ __forceinline__ bool status_open(u32 s) { return s >= kStatusLink; }
 
 __device__ __forceinline__ u64 request_index(const batch_args& a, u64 i) {
   return a.perm_mul ? (a.perm_lo + i) * a.perm_mul % a.perm_n : i;
@@ -146,12 +158,14 @@ batch_kernel(tree_view tv, batch_args a) {
   op_state<gpu_node> st;
   request rq;
   // with skip_finds, the tile's first 16 lanes look at the next 16 requests the tile
-  // would take and it moves to the first that is not a find
+  // would take and it moves to the first that is not a find; with statuses, to the first
+  // that is open
   auto seek = [&]() {
-    if (!a.skip_finds || !a.types) return;
+    if (!a.status && (!a.skip_finds || !a.types)) return;
     while (i < hi) {
       const u64 e = i + (u64)c.slot * ntiles;
-      const u32 m = c.ballot(e < hi && a.types[request_index(a, e)] != op_find);
+      const u32 m = c.ballot(e < hi && (a.status ? status_open(a.status[e - lo])
+                                                 : a.types[request_index(a, e)] != op_find));
       if (m) {
         i += (u64)(__ffs(m) - 1) * ntiles;
         return;
@@ -167,19 +181,23 @@ batch_kernel(tree_view tv, batch_args a) {
     const bool writes = rq.kind == op_insert || rq.kind == op_update || rq.kind == op_upsert;
     const bool bad_len = rq.key_length == 0 || rq.key_length > a.max_key_length ||
                          (writes && rq.value_length > a.max_value_length);
-    if (bad_len) rq.key_length = 0;  // nothing of the request is read
+    const bool link = a.status && a.status[i - lo] == kStatusLink;
+    if (link) rq.kind = op_link;
+    if (bad_len || link) rq.key_length = 0;  // nothing of the request is read
     c.load_key_cache(rq);
     op_begin(c, st, tv.root);
-    if (a.hints && rq.kind != op_find && !bad_len) {
+    if (a.hints && rq.kind != op_find && (link || !bad_len)) {
       // start at the border node the read-only pass reached (B-link: a node that split
       // since is left by moving right; one that became interior is descended)
       const u32* hp = a.hints + (u64)kHintWords * (i - lo);
       const u32 hn = hp[0], hr = hp[1], hpar = hp[2], hl = hp[3];
       const u32 ns = tv.pool.num_slabs;
-      if (hn < ns && hr < ns && hl < rq.key_length)
+      if (link)
+        op_begin_link(st, hn, hr, hpar, hl < ns ? hl : kInvalid);
+      else if (hn < ns && hr < ns && hl < rq.key_length)
         op_begin_at(st, hn, hr, hpar < ns ? hpar : kInvalid, hl);
     }
-    if (bad_len) {
+    if (bad_len && !link) {
       c.set_error(kErrBadLength);
       op_finish(st, 0);
     } else if (abort_pending(tv.err)) {
@@ -215,7 +233,7 @@ batch_kernel(tree_view tv, batch_args a) {
       if (c.lane == 0) {
         if (rq.kind == op_find) {
           if (a.out_value_lengths) a.out_value_lengths[ri] = st.result;
-        } else if (a.results) {
+        } else if (a.results && rq.kind != op_link) {
           a.results[ri] = st.result != 0;
         }
       }
@@ -842,12 +860,31 @@ __global__ void __launch_bounds__(kBlockThreads) scan_kernel(tree_view tv, scan_
 }
 
 // ---------------------------------------------------------------------------------
-__global__ void drain_kernel(slab_pool_view pool, retire_view rv) {
-  const u32 raw = *rv.count;
-  const u32 count = raw < rv.capacity ? raw : rv.capacity;
+// Frees what a launch retired.  With statuses (of n positions) it also reports what the
+// grouped writes decided and frees the records they replaced: the one pass in launch order
+// takes the place of a scattered byte store and a retire-list entry per request.
+__global__ void drain_kernel(slab_pool_view pool, retire_view rv, batch_args a, u32 n) {
   const u32 stride = gridDim.x * blockDim.x;
-  for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride)
-    dev::free_retired(pool, rv.list[i]);
+  const u32 first = blockIdx.x * blockDim.x + threadIdx.x;
+  if (rv.enabled) {
+    const u32 raw = *rv.count;
+    const u32 count = raw < rv.capacity ? raw : rv.capacity;
+    for (u32 i = first; i < count; i += stride) dev::free_retired(pool, rv.list[i]);
+  }
+  if (!a.status) return;
+  u64 lo = 0;
+  if (a.range) {
+    const u64 hi = min(a.range[1], a.n);
+    lo = min(a.range[0], hi);
+    n = (u32)min((u64)n, hi - lo);
+  }
+  for (u32 p = first; p < n; p += stride) {
+    const u32 s = a.status[p];
+    if (s == kStatusOpen || s == kStatusNone) continue;
+    if (a.results) a.results[request_index(a, lo + p)] = s != kStatusFail;
+    if (rv.enabled && s >= kStatusRecord && s < kStatusRecord + kMaxPoolSlabs)
+      dev::free_retired(pool, s & ~kStatusRecord);
+  }
 }
 
 __global__ void set_error_kernel(u32* err, u32 code) { dev::set_error(err, code); }

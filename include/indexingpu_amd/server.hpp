@@ -472,7 +472,8 @@ class masstree_server {
 
   void drain_list(int l, serve_stats& st) {
     const retire_view rv = lists_[l].rec->get_device_instance();
-    hipLaunchKernelGGL(drain_kernel, dim3(256), dim3(256), 0, aux_, tree_.allocator_, rv);
+    hipLaunchKernelGGL(drain_kernel, dim3(256), dim3(256), 0, aux_, tree_.allocator_, rv,
+                       batch_args{}, 0u);
     hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(64), 0, aux_, rv);
     IGPU_HIP_TRY(hipEventRecord(aux_ev_, aux_));
     st.drains++;

@@ -47,6 +47,9 @@ enum op_kind : u32 {
   op_find = 2,
   op_update = 3,
   op_upsert = 4,  // insert<update_if_exists=true>
+  // not a request (request types are bytes): links a right node, split off and reachable
+  // only through its left neighbour, into its parent (op_begin_link)
+  op_link = 0x100,
 };
 
 enum op_phase : u32 {
@@ -225,6 +228,34 @@ IGPU_HD void op_begin_at(S& st, u32 node, u32 layer_root, u32 parent, u32 layer)
   st.layer_root = layer_root;
   st.hint[0] = parent;
   st.lvl = 0;
+}
+
+// Starts (an operation already begun) the link of border node `right` of the layer rooted
+// at `layer_root` into its parent, with the separator `sep` that is its left neighbour's
+// high key; `parent` is a level-1 node at or left of that parent (kInvalid: unknown).  It
+// holds no locks (a0 = kInvalid: no child node of it, so ph_parent_lock places the link at
+// the slot that covers the separator).  The links of several right nodes of one split node
+// may be made in any order, beside further splits of any of them: the covering slot always
+// names a node at or left of the one the separator bounds, which B-link move-right passes.
+template <class S>
+IGPU_HD void op_begin_link(S& st, u32 right, u32 sep, u32 layer_root, u32 parent) {
+  st.layer_root = layer_root;
+  st.hint[0] = parent;
+  st.a0 = kInvalid;
+  st.a1 = right;
+  st.a2 = sep;
+  st.a3 = 1;
+  st.result = 1;
+  goto_parent(st);
+}
+
+// Publishes the two halves of a split whose separator has been placed (or cannot be); a
+// link (op_begin_link) holds none.
+template <class C, class S>
+IGPU_HD void publish_halves(C& c, const S& st) {
+  if (st.a0 == kInvalid) return;
+  c.unlock_bump(st.a0);
+  c.unlock_bump(st.a1);
 }
 
 template <class S>
@@ -408,8 +439,7 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
         // a split waiting for its parent holds both halves (written, not yet
         // published); publish them: the right half is reachable through the left
         // one's sibling link, and a later split of it links it from its left neighbour
-        c.unlock_bump(st.a0);
-        c.unlock_bump(st.a1);
+        publish_halves(c, st);
       } else if (op_in_merge(st)) {
         c.unlock_bump(st.a0);  // the emptied node stays, empty and linked
       } else if (op_holds_locks(st)) {
@@ -785,8 +815,7 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
         c.interior_insert(n, j, st.a2, lc, st.a1);
         c.write_node(st.node, n);
         c.unlock_bump(st.node);
-        c.unlock_bump(st.a0);
-        c.unlock_bump(st.a1);
+        publish_halves(c, st);
         op_finish(st, st.result);
         return true;
       }
@@ -799,8 +828,7 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
           // reachable through the sibling link, so every route is still correct, and a
           // later split of it links it from its left neighbour's slot (above).
           c.unlock_same(st.node);
-          c.unlock_bump(st.a0);
-          c.unlock_bump(st.a1);
+          publish_halves(c, st);
           op_finish(st, st.result);
           return true;
         }
@@ -815,16 +843,14 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
         c.make_interior_root(n, sep2, li, ri, st.a3 + 1, h);
         c.write_node(st.node, n);
         c.unlock_bump(st.node);
-        c.unlock_bump(st.a0);
-        c.unlock_bump(st.a1);
+        publish_halves(c, st);
         op_finish(st, st.result);
         return true;
       }
       const u32 ri = c.alloc_slab();
       if (ri == kInvalid) {
         c.unlock_same(st.node);
-        c.unlock_bump(st.a0);
-        c.unlock_bump(st.a1);
+        publish_halves(c, st);
         op_finish(st, st.result);
         return true;
       }
@@ -836,8 +862,7 @@ IGPU_HD bool op_step(C& c, const request& rq, S& st) {
       c.write_node(ri, right);
       c.write_node(st.node, left);
       c.fence_release();
-      c.unlock_bump(st.a0);
-      c.unlock_bump(st.a1);
+      publish_halves(c, st);
       st.a0 = st.node;
       st.a1 = ri;
       st.a2 = sep2;

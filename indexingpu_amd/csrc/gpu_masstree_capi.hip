@@ -409,6 +409,12 @@ int gmt_set_write_hints(gmt_index* index, uint32_t min_requests) {
   return GMT_OK;
 }
 
+int gmt_set_write_groups(gmt_index* index, uint32_t min_requests) {
+  if (!index) return bad("gmt_set_write_groups: null handle");
+  B(index)->on_all([&](auto& t) { t.set_write_groups(min_requests); });
+  return GMT_OK;
+}
+
 int gmt_set_mixed_split(gmt_index* index, uint32_t min_requests) {
   if (!index) return bad("gmt_set_mixed_split: null handle");
   B(index)->on_all([&](auto& t) { t.set_mixed_split(min_requests); });

@@ -86,6 +86,7 @@ def load_library():
     lib.gmt_set_record_tile.argtypes = [vp, u32]
     lib.gmt_set_mixed_split.argtypes = [vp, u32]
     lib.gmt_set_write_hints.argtypes = [vp, u32]
+    lib.gmt_set_write_groups.argtypes = [vp, u32]
     lib.gmt_reserve_find_scratch.argtypes = [vp, ctypes.c_uint64]
     lib.gmt_tile_size.argtypes = [vp]
     lib.gmt_tile_size.restype = u32
@@ -349,6 +350,12 @@ class GpuMasstree:
         """Insert, update and erase batches of at least min_requests requests start their
         writes at border nodes found by a read-only descent (0xFFFFFFFF: never)."""
         self._check(self._lib.gmt_set_write_hints(self._h, int(min_requests) & 0xFFFFFFFF))
+
+    def set_write_groups(self, min_requests):
+        """Hinted write batches of at least min_requests requests, and split mixed batches of
+        at least twice as many, apply their writes border node by border node (0xFFFFFFFF:
+        never)."""
+        self._check(self._lib.gmt_set_write_groups(self._h, int(min_requests) & 0xFFFFFFFF))
 
     def reserve_find_scratch(self, max_requests):
         """Allocates the two-pass find scratch for batches of up to max_requests requests
