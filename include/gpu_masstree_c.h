@@ -193,7 +193,7 @@ int gmt_set_find_passes(gmt_index* index, uint32_t passes);
  * do not depend on it. */
 int gmt_set_record_tile(gmt_index* index, uint32_t record_tile);
 
-/* Mixed batches of at least min_requests requests (default 8192) run their finds as a
+/* Mixed batches of at least min_requests requests (default 16384) run their finds as a
  * read-only pass with the narrow two-pass kernels, then the other requests; 0 splits
  * every batch, 0xFFFFFFFF none.  The first split batch at a new largest size allocates
  * 4 bytes per request of scratch and synchronizes.  A tuning knob with no counterpart in

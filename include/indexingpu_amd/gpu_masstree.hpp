@@ -890,7 +890,8 @@ struct gpu_masstree {
   // nodes, where they serialize on the locks and on the coherent reads of those lines
   // (16M keys into an empty tree: 13 Mops/s in one launch, ~500 Mops/s in growing
   // launches).  The batch therefore runs as consecutive launches that each grow the
-  // tree at most kGrowthFactor-fold (from kGrowthMin keys), then the rest in one launch.
+  // tree at most kGrowthFactor-fold (from kGrowthMin keys; by kGrowthGrouped once their
+  // writes are grouped), then the rest in one launch.
   // The launches take the requests in a scattered order (index times a multiplier coprime to n, modulo n), so
   // each one is a sample of the whole batch: a batch in key order -- or one whose keys
   // all lie past the tree's current right edge -- then grows every key range at once
@@ -900,7 +901,13 @@ struct gpu_masstree {
   // bounds how spread out the tree is).
   static constexpr uint64_t kGrowthMin = 512;
   static constexpr uint64_t kGrowthFactor = 4;
-  static constexpr uint64_t kGrowthGrouped = 2;  // stages that run as grouped writes
+  // Stages that run as grouped writes grow the tree by a half: a node of ten entries then
+  // gets five more on average, and next to none gets more than a tile applies or two nodes
+  // hold.  At twice the tree a twentieth of the requests were left to the step machine, all
+  // on nodes that split: 16M keys loaded (and found) in 21.2 ms, by halves in 20.7, by thirds
+  // in 22.4.  Stages use a shortcut table that is there but build none: a build in each (a
+  // host wait and up to 0.6 ms) gave less than it took, 20.7 against 19.0 ms.
+  static constexpr uint64_t kGrowthGrouped = 2;
   // Weyl multiplier: the integer nearest n / golden ratio that is coprime to n, so
   // j -> j * m mod n is a bijection and any run of consecutive j lands spread evenly
   // over [0, n) (three-gap theorem).
@@ -926,7 +933,7 @@ struct gpu_masstree {
     auto room = [&]() {
       const bool grouped = write_group_min_ != 0xFFFFFFFFu && size >= write_group_min_;
       return std::max<uint64_t>(kGrowthMin,
-                                size * ((grouped ? kGrowthGrouped : kGrowthFactor) - 1));
+                                grouped ? size / kGrowthGrouped : size * (kGrowthFactor - 1));
     };
     if (room() >= n) {
       launch_hinted(a, stream);  // the tree is large enough: no growth stages
@@ -949,8 +956,8 @@ struct gpu_masstree {
       indexingpu_amd::batch_args s = a;
       s.perm_lo = done;
       s.n = stage;
-      *inserted_hint_ = size;  // the stage's hint descent may use a shortcut table
-      launch_hinted(s, stream);
+      *inserted_hint_ = size;
+      launch_hinted(s, stream, false);
       done += stage;
       size += stage;
     }
@@ -965,7 +972,8 @@ struct gpu_masstree {
   // left by moving right).  The requests of a batch are independent, so chunks give
   // the results of one launch.
   static constexpr uint64_t kHintChunk = 1ull << 22;
-  void launch_hinted(const indexingpu_amd::batch_args& a, hipStream_t stream) {
+  void launch_hinted(const indexingpu_amd::batch_args& a, hipStream_t stream,
+                     bool refresh = true) {
     const uint64_t n = a.n;
     if (n == 0) return;
     if (write_hint_min_ == 0xFFFFFFFFu || n < write_hint_min_) {
@@ -973,7 +981,7 @@ struct gpu_masstree {
       return;
     }
     ensure_hints(std::min<uint64_t>(n, kHintChunk));
-    refresh_shortcut(stream);
+    if (refresh) refresh_shortcut(stream);
     for (uint64_t off = 0; off < n; off += kHintChunk) {
       indexingpu_amd::batch_args c = a;
       c.n = std::min<uint64_t>(kHintChunk, n - off);
@@ -994,7 +1002,7 @@ struct gpu_masstree {
         case 16: launch_descend_only<16>(c, stream); break;
         default: launch_descend_only<2>(c, stream); break;
       }
-      launch_groups(c, c.n, stream);
+      launch_groups(c, c.n, stream, a.kind == indexingpu_amd::op_insert ? off : 0);
       launch_batch<true>(c, stream, true);
     }
   }
@@ -1007,12 +1015,16 @@ struct gpu_masstree {
   // mixed batches of n requests, a tenth of them writes: 16K 93 / 88 us, 32K 104 / 109,
   // 64K 116 / 158.
   static constexpr uint64_t kMaxGroupSlots = 1ull << 23;
-  void launch_groups(indexingpu_amd::batch_args& a, uint64_t n, hipStream_t stream) {
+  static constexpr uint64_t kLinkShare = 4;
+  // `added`: keys that earlier launches of the batch may have inserted.
+  void launch_groups(indexingpu_amd::batch_args& a, uint64_t n, hipStream_t stream,
+                     uint64_t added = 0) {
     // of a mixed batch half the requests are taken to write
     if (write_group_min_ == 0xFFFFFFFFu || (a.types ? n / 2 : n) < write_group_min_ ||
         n >= (1ull << 31))
       return;
-    const group_size shape = group_shape(n, *inserted_hint_, a.types != nullptr);
+    const uint64_t size = *inserted_hint_ + added;
+    const group_size shape = group_shape(n, size, a.types != nullptr);
     if (!ensure_groups(n, shape, stream)) return;
     a.flags |= fanout_flags_;
     const uint32_t threads = indexingpu_amd::kBlockThreads;
@@ -1040,9 +1052,21 @@ struct gpu_masstree {
     hipLaunchKernelGGL(build, grid(n, build), dim3(threads), 0, stream, a, g, allocator_);
     hipLaunchKernelGGL(write, writers, dim3(threads), 0, stream, view(), a, g);
     a.status = group_status_;
+    // Links by parents where most parents get some: a batch of a quarter of the tree or more
+    // (stages are halves).  Per stage of a 1M-key load the two launches take 15 to 60 us and
+    // batch_kernel 270 -> 40 us less than that; a 4M batch on 16M keys makes few links.
+    if (stores && a.kind != indexingpu_amd::op_update && !a.types &&
+        n * kLinkShare >= size) {
+      auto build_links = indexingpu_amd::group_link_build_kernel;
+      auto link = indexingpu_amd::group_link_kernel;
+      hipLaunchKernelGGL(build_links, grid(n, build_links), dim3(threads), 0, stream, a, g,
+                         allocator_.num_slabs);
+      hipLaunchKernelGGL(link, grid(shape.slots / window * 64, link), dim3(threads), 0, stream,
+                         view(), a, g);
+    }
   }
   // The table for n positions over a tree of `size` keys: a slot for every border node that
-  // may be written (ten keys fill one on average; of a mixed batch half the requests are
+  // may be written (eight to ten keys fill one; of a mixed batch half the requests are
   // taken to write), each with room for three times the average requests of a node (4 to
   // 16), 512 MB in all at most.  What does not fit is left to batch_kernel.
   struct group_size {
@@ -1051,7 +1075,7 @@ struct gpu_masstree {
   static constexpr uint64_t kMaxGroupRooms = 1ull << 25;
   static group_size group_shape(uint64_t n, uint64_t size, bool mixed) {
     const uint64_t writes = mixed ? n / 2 : n;
-    const uint64_t nodes = std::max<uint64_t>(64, std::min<uint64_t>(writes, size / 10));
+    const uint64_t nodes = std::max<uint64_t>(64, std::min<uint64_t>(writes, size / 8));
     group_size g{64, 4};
     while (g.slots * 20 < nodes * 23 && g.slots < kMaxGroupSlots) g.slots *= 2;
     while (g.room < indexingpu_amd::kGroupTake && g.room * nodes < 3 * writes &&

@@ -58,6 +58,31 @@ __device__ __forceinline__ u64 launch_range(const batch_args& a, u64& lo) {
   return hi;
 }
 
+// Adds a request to the slot of `node`, if there is room.
+__device__ __forceinline__ void group_join(const group_view& g, u32 node, const uint4& req) {
+  const u32 mask = g.slots - 1;
+  u32 h = (node * 0x9E3779B1u) >> 7 & mask;
+  for (u32 probe = 0; probe < kGroupProbes; probe++, h = (h + 1) & mask) {
+    const u64 cur = dev::coherent_load(g.heads + h);
+    u32* head = reinterpret_cast<u32*>(g.heads + h);
+    u32 at = slot_lo(cur);
+    if (at == 0) {
+      u32 expected = 0;
+      at = __hip_atomic_compare_exchange_strong(head, &expected, node + 1, __ATOMIC_RELAXED,
+                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+               ? node + 1
+               : expected;
+    }
+    if (at == node + 1) {
+      if (slot_hi(cur) < g.room) {
+        const u32 r = dev::atomic_add(head + 1, 1u);
+        if (r < g.room) g.body[(u64)h * g.room + r] = req;
+      }
+      return;
+    }
+  }
+}
+
 // Bound by the table's random lines: a load, a compare-and-swap for the first request of a
 // node, an add and the request's 16 bytes.  It reads what the groups need of each request in
 // launch order, so group_write_kernel gathers key and value rows only.  A node that more
@@ -72,7 +97,6 @@ __global__ void __launch_bounds__(kBlockThreads) group_build_kernel(batch_args a
   u64 lo;
   const u64 hi = launch_range(a, lo);
   const u32 n = (u32)(hi - lo);
-  const u32 mask = g.slots - 1;
   const u32 stride = gridDim.x * kBlockThreads;
   const u32 maxK = a.max_key_length, maxV = a.max_value_length;
   for (u32 p0 = blockIdx.x * kBlockThreads; p0 < n; p0 += stride) {
@@ -104,28 +128,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_build_kernel(batch_args a
       const u32 first = (u32)__builtin_amdgcn_readlane((int)node, __ffsll((unsigned long long)have) - 1);
       if ((u32)__popcll(__ballot(node == first)) > kGroupTake && node == first) node = kInvalid;
     }
-    if (node != kInvalid) {
-      u32 h = (node * 0x9E3779B1u) >> 7 & mask;
-      for (u32 probe = 0; probe < kGroupProbes; probe++, h = (h + 1) & mask) {
-        const u64 cur = dev::coherent_load(g.heads + h);
-        u32* head = reinterpret_cast<u32*>(g.heads + h);
-        u32 at = slot_lo(cur);
-        if (at == 0) {
-          u32 expected = 0;
-          at = __hip_atomic_compare_exchange_strong(head, &expected, node + 1, __ATOMIC_RELAXED,
-                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                   ? node + 1
-                   : expected;
-        }
-        if (at == node + 1) {
-          if (slot_hi(cur) < g.room) {
-            const u32 r = dev::atomic_add(head + 1, 1u);
-            if (r < g.room) g.body[(u64)h * g.room + r] = req;
-          }
-          break;
-        }
-      }
-    }
+    if (node != kInvalid) group_join(g, node, req);
     if (p < n) g.status[p] = status;
   }
 }
@@ -597,6 +600,154 @@ __global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv
           status = kStatusLink;
         }
         g.status[p] = status;
+      }
+    }
+  }
+  unlock();
+  if (ws.bits != 0 && lane64 == 0) dev::atomic_and(&tv.pool.bitmap[ws.word], ~ws.bits);
+}
+
+// Links of new border nodes, grouped by their level-1 parents as the writes are by border
+// node (the table is empty again): body entries are position, separator, right node, layer
+// root.  For batches that split a node of most parents: there the step machine's tiles
+// queued on the parents' locks (0.3 ms in every growth stage of a load, 1.2 ms where a
+// stage splits 450K nodes).
+__global__ void __launch_bounds__(kBlockThreads) group_link_build_kernel(batch_args a,
+                                                                          group_view g,
+                                                                          u32 num_slabs) {
+  u64 lo;
+  const u64 hi = launch_range(a, lo);
+  const u32 n = (u32)(hi - lo);
+  for (u32 p = blockIdx.x * kBlockThreads + threadIdx.x; p < n; p += gridDim.x * kBlockThreads) {
+    if (g.status[p] != kStatusLink) continue;
+    const uint4 hint = *reinterpret_cast<const uint4*>(a.hints + (u64)kHintWords * p);
+    if (hint.w < num_slabs) group_join(g, hint.w, make_uint4(p, hint.y, hint.x, hint.z));
+  }
+}
+
+// One tile merges up to 16 links into their parent, in one or two nodes.  A node is taken as
+// (low bound, child) items: a link is the item (separator, right node), and the upper bound
+// of each item is the next one's low bound.  Bound by latency, as group_write_kernel.
+__global__ void __launch_bounds__(kBlockThreads) group_link_kernel(tree_view tv, batch_args a,
+                                                                    group_view g) {
+  const wave_tile<16, true> c(tv.pool, tv.retire, tv.err, tv.root);
+  const u32 lane64 = threadIdx.x & 63u, slot = c.slot, tile = lane64 >> 4;
+  const u32 below_me = (1u << slot) - 1u;
+  const u32 cap_bits = (a.flags >> kReqInteriorCapShift) & 15u;
+  const u32 cap = cap_bits ? cap_bits : kInteriorCap;
+  const u32 version_mask = ~((1u << kVersionShift) - 1u);
+  __shared__ u64 items[kBlockThreads / 16][32];  // a tile's (low bound, child), in order
+  u64* const it = items[threadIdx.x / 16];
+  wave_slabs ws;
+  u32 unlock_node = kInvalid, unlock_to = 0;  // as in group_write_kernel
+  auto unlock = [&]() {
+    dev::order();
+    if (unlock_node != kInvalid) dev::coherent_store(c.hdr_ptr(unlock_node), unlock_to);
+    unlock_node = kInvalid;
+  };
+  const bool in_window = lane64 < g.window;
+  for (u32 w0 = (blockIdx.x * (kBlockThreads / 64) + threadIdx.x / 64) * g.window; w0 < g.slots;
+       w0 += gridDim.x * (kBlockThreads / 64) * g.window) {
+    const u64 entry = in_window ? g.heads[w0 + lane64] : 0ull;
+    u64 todo = __ballot(slot_lo(entry) != 0);
+    if (slot_lo(entry) != 0) g.heads[w0 + lane64] = 0;
+    while (todo) {
+      u32 from_slot = 64;
+#pragma unroll
+      for (u32 t = 0; t < 4; t++) {
+        if (todo == 0) break;
+        if (tile == t) from_slot = (u32)__ffsll((unsigned long long)todo) - 1u;
+        todo &= todo - 1;
+      }
+      const u32 node = __shfl(slot_lo(entry), (int)(from_slot & 63u), 64) - 1u;
+      const u32 joined = __shfl(slot_hi(entry), (int)(from_slot & 63u), 64);
+      const bool live = from_slot < 64 && node < tv.pool.num_slabs;
+      const u32 k = live ? min(joined, g.room) : 0u;
+      gpu_node nd;
+      nd.s = live ? c.slab(node)[slot] : 0ull;
+      const bool have = slot < k;
+      uint4 req = make_uint4(0, 0, 0, 0);
+      if (have) req = g.body[(u64)(w0 + from_slot) * g.room + slot];
+      unlock();
+      const u32 sep = req.y;
+      const u32 h = c.header(nd), sib = c.sibling(nd);
+      const bool usable = live && !hdr_border(h) && !hdr_locked(h) && hdr_level(h) == 1 &&
+                          hdr_nkeys(h) >= 1 && hdr_nkeys(h) <= kInteriorCap;
+      const u32 nk = usable ? hdr_nkeys(h) : 0u;
+      const bool is_child = slot < nk;
+      const u32 bound = slot_lo(nd.s), child = slot_hi(nd.s) & kChildMask;
+      const u32 high = c.bcast(bound, nk ? nk - 1 : 0u);
+      const u32 before = c.bcast(bound, slot ? slot - 1 : 0u);  // the low bound of child `slot`
+      // ---- which links, and their order among the bounds and each other
+      bool ok = usable && have && sep < high;
+      u32 bounds_below = 0, links_below = 0;  // link lane: bounds, links below its separator
+      u32 links_under = 0;                    // child lane: links below its low bound
+      for (u32 r = 0; __ballot(r < k); r++) {
+        const u32 s = c.bcast(sep, r), on = c.bcast(ok ? 1u : 0u, r);
+        const u32 lt = c.ballot(is_child && bound < s), eq = c.ballot(is_child && bound == s);
+        if (r >= k || !on) continue;
+        if (slot == r) {
+          bounds_below = (u32)__popc(lt);
+          if (eq) ok = false;  // not expected: a separator lies inside its node's range
+        }
+        if (ok && slot > r && sep == s) ok = false;
+        if (sep > s) links_below |= 1u << r;
+        if (slot > 0 && before > s) links_under |= 1u << r;
+      }
+      u32 okm = c.ballot(ok);
+      // two nodes at most; a layer root splits in place, which is left to batch_kernel
+      const u32 room = (hdr_root(h) ? cap : 2 * cap);
+      if (ok && nk + (u32)__popc(okm & below_me) >= room) ok = false;
+      okm = c.ballot(ok);
+      u32 T = nk + (u32)__popc(okm);
+      const bool wants = okm && T > cap;
+      const u32 fresh = c.bcast(wave_alloc(tv.pool, ws, 1, wants && slot == 0), 0);
+      if (wants && fresh == kInvalid) {  // out of slabs: what fits
+        if (ok && nk + (u32)__popc(okm & below_me) >= cap) ok = false;
+      }
+      okm = c.ballot(ok);
+      T = nk + (u32)__popc(okm);
+      const bool changed = okm != 0;
+      const bool split = changed && wants && fresh != kInvalid;
+      if (changed && slot == kMetaSlot) dev::coherent_store(c.hdr_ptr(node), h | kLockBit);
+      it[slot] = 0;
+      it[slot + 16] = 0;
+      lds_order();
+      if (is_child) it[slot + (u32)__popc(links_under & okm)] = slot_make(slot ? before : 0u, child);
+      if (ok) it[1 + bounds_below + (u32)__popc(links_below & okm)] = slot_make(sep, req.z);
+      lds_order();
+      const u32 cut = split ? T / 2 : T;
+      const u32 cut_low = slot_lo(it[cut & 31u]);  // the left node's last bound, in a split
+      const u64 own = it[slot], next = it[slot + 1];
+      const u64 rown = it[(cut + slot) & 31u], rnext = it[(cut + slot + 1) & 31u];
+      dev::order();  // the lock is stored
+      auto line = [&](u64 mine, u64 after, u32 count, u32 last, u32 header, u32 sibling) -> u64 {
+        u64 v = 0;
+        if (slot < count) v = slot_make(slot + 1 < count ? slot_lo(after) : last, slot_hi(mine));
+        if (slot == kMetaSlot) v = slot_make(header, sibling);
+        if (slot < kTagSlots) v |= (u64)((hdr_publish_tag(header) >> slot) & 1u) << 63;
+        return v;
+      };
+      if (split)
+        dev::coherent_store(c.slab(fresh) + slot,
+                            line(rown, rnext, T - cut, high, hdr_make(T - cut, false, false, 1), sib));
+      if (changed) {
+        const u32 lh = hdr_with_nkeys(h, cut) | kLockBit;
+        dev::coherent_store(c.slab(node) + slot,
+                            line(own, next, cut, split ? cut_low : high, lh, split ? fresh : sib));
+        if (slot == kMetaSlot) {
+          unlock_node = node;
+          unlock_to = hdr_unlocked_next(lh);
+        }
+      }
+      if (have && ok) {
+        u32 status = kStatusDone;
+        if (split && (okm & below_me) == 0) {
+          *reinterpret_cast<uint4*>(a.hints + (u64)kHintWords * req.x) =
+              make_uint4(fresh, cut_low, req.w, kInvalid);
+          status = kStatusLinkUp;
+        }
+        g.status[req.x] = status;
       }
     }
   }

@@ -103,11 +103,12 @@ constexpr u32 kHintWords = 4;
 // Statuses of launch positions (group_write.hpp).
 constexpr u32 kStatusOpen = 0xFFFFFFFFu;    // left to batch_kernel
 constexpr u32 kStatusLink = 0xFFFFFFFEu;    // succeeded; its hint words hold a link (op_link)
-constexpr u32 kStatusDone = 0xFFFFFFFDu;    // succeeded
-constexpr u32 kStatusFail = 0xFFFFFFFCu;    // failed (stored already, or absent)
-constexpr u32 kStatusNone = 0xFFFFFFFBu;    // not a write
+constexpr u32 kStatusLinkUp = 0xFFFFFFFDu;  // the same, of a level-1 node into level 2
+constexpr u32 kStatusDone = 0xFFFFFFFCu;    // succeeded
+constexpr u32 kStatusFail = 0xFFFFFFFBu;    // failed (stored already, or absent)
+constexpr u32 kStatusNone = 0xFFFFFFFAu;    // not a write
 constexpr u32 kStatusRecord = 0x80000000u;  // succeeded; bits 0-30: the record it replaced
-__device__ __forceinline__ bool status_open(u32 s) { return s >= kStatusLink; }
+__device__ __forceinline__ bool status_open(u32 s) { return s >= kStatusLinkUp; }
 
 __device__ __forceinline__ u64 request_index(const batch_args& a, u64 i) {
   return a.perm_mul ? (a.perm_lo + i) * a.perm_mul % a.perm_n : i;
@@ -181,7 +182,8 @@ batch_kernel(tree_view tv, batch_args a) {
     const bool writes = rq.kind == op_insert || rq.kind == op_update || rq.kind == op_upsert;
     const bool bad_len = rq.key_length == 0 || rq.key_length > a.max_key_length ||
                          (writes && rq.value_length > a.max_value_length);
-    const bool link = a.status && a.status[i - lo] == kStatusLink;
+    const u32 status = a.status ? a.status[i - lo] : kStatusOpen;
+    const bool link = status != kStatusOpen;
     if (link) rq.kind = op_link;
     if (bad_len || link) rq.key_length = 0;  // nothing of the request is read
     c.load_key_cache(rq);
@@ -193,7 +195,7 @@ batch_kernel(tree_view tv, batch_args a) {
       const u32 hn = hp[0], hr = hp[1], hpar = hp[2], hl = hp[3];
       const u32 ns = tv.pool.num_slabs;
       if (link)
-        op_begin_link(st, hn, hr, hpar, hl < ns ? hl : kInvalid);
+        op_begin_link(st, hn, hr, hpar, hl < ns ? hl : kInvalid, status == kStatusLink ? 1u : 2u);
       else if (hn < ns && hr < ns && hl < rq.key_length)
         op_begin_at(st, hn, hr, hpar < ns ? hpar : kInvalid, hl);
     }

@@ -230,21 +230,22 @@ IGPU_HD void op_begin_at(S& st, u32 node, u32 layer_root, u32 parent, u32 layer)
   st.lvl = 0;
 }
 
-// Starts (an operation already begun) the link of border node `right` of the layer rooted
-// at `layer_root` into its parent, with the separator `sep` that is its left neighbour's
-// high key; `parent` is a level-1 node at or left of that parent (kInvalid: unknown).  It
-// holds no locks (a0 = kInvalid: no child node of it, so ph_parent_lock places the link at
-// the slot that covers the separator).  The links of several right nodes of one split node
-// may be made in any order, beside further splits of any of them: the covering slot always
-// names a node at or left of the one the separator bounds, which B-link move-right passes.
+// Starts (an operation already begun) the link of node `right` (on the level below `level`,
+// of the layer rooted at `layer_root`) into its parent, with the separator `sep` that bounds
+// its left neighbour; `parent` is a node of `level` at or left of that parent (kInvalid:
+// unknown).  It holds no locks (a0 = kInvalid: no child node of it, so ph_parent_lock places
+// the link at the slot that covers the separator).  The links of several right nodes of one
+// split node may be made in any order, beside further splits of any of them: the covering
+// slot always names a node at or left of the one the separator bounds, which B-link
+// move-right passes.
 template <class S>
-IGPU_HD void op_begin_link(S& st, u32 right, u32 sep, u32 layer_root, u32 parent) {
+IGPU_HD void op_begin_link(S& st, u32 right, u32 sep, u32 layer_root, u32 parent, u32 level = 1) {
   st.layer_root = layer_root;
-  st.hint[0] = parent;
+  st.hint[level - 1] = parent;
   st.a0 = kInvalid;
   st.a1 = right;
   st.a2 = sep;
-  st.a3 = 1;
+  st.a3 = level;
   st.result = 1;
   goto_parent(st);
 }
