@@ -947,7 +947,7 @@ struct gpu_masstree {
     if (write_hint_min_ != 0xFFFFFFFFu && n >= write_hint_min_) {
       ensure_hints(chunk);
       if (write_group_min_ != 0xFFFFFFFFu && n >= write_group_min_)
-        ensure_groups(chunk, group_shape(chunk, size + n, false), stream);
+        ensure_groups(chunk, group_shape(chunk, (size + n) / 3 * 2, false), stream);
     }
     uint64_t done = 0;
     while (done < n) {
@@ -1016,6 +1016,7 @@ struct gpu_masstree {
   // 64K 116 / 158.
   static constexpr uint64_t kMaxGroupSlots = 1ull << 23;
   static constexpr uint64_t kLinkShare = 4;
+  static constexpr uint64_t kMaxDealtWords = 32;
   // `added`: keys that earlier launches of the batch may have inserted.
   void launch_groups(indexingpu_amd::batch_args& a, uint64_t n, hipStream_t stream,
                      uint64_t added = 0) {
@@ -1041,10 +1042,12 @@ struct gpu_masstree {
     const uint64_t most_waves = (uint64_t)indexingpu_amd::resident_blocks(write) * (threads / 64);
     uint32_t window = 64;
     while (window > 4 && shape.slots / window < most_waves) window /= 2;
-    const dim3 writers = grid(shape.slots / window * 64, write);
-    // a wave steps the claim cursor about twice in the launch, for 16 bitmap words at most
-    const uint32_t words = (uint32_t)std::max<uint64_t>(
-        1, std::min<uint64_t>(16, (a.types ? n / 2 : n) / (64 * (threads / 64) * writers.x)));
+    const dim3 writers = grid((shape.slots + window - 1) / window * 64, write);
+    // most of the bitmap words the launch may need are dealt to the waves beforehand (of a
+    // mixed batch, of which few may be inserts, one each)
+    const uint64_t per_wave = n / (32 * (threads / 64) * (uint64_t)writers.x);
+    const uint32_t words = a.types ? 1u : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(
+                                               kMaxDealtWords, per_wave * 3 / 4));
     const indexingpu_amd::group_view g{
         group_heads_, reinterpret_cast<uint4*>(group_body_), (uint32_t)shape.slots,
         (uint32_t)shape.room, group_status_, reinterpret_cast<uint32_t*>(group_heads_ + group_slots_),
@@ -1061,14 +1064,15 @@ struct gpu_masstree {
       auto link = indexingpu_amd::group_link_kernel;
       hipLaunchKernelGGL(build_links, grid(n, build_links), dim3(threads), 0, stream, a, g,
                          allocator_.num_slabs);
-      hipLaunchKernelGGL(link, grid(shape.slots / window * 64, link), dim3(threads), 0, stream,
+      hipLaunchKernelGGL(link, grid((shape.slots + window - 1) / window * 64, link), dim3(threads), 0, stream,
                          view(), a, g);
     }
   }
   // The table for n positions over a tree of `size` keys: a slot for every border node that
-  // may be written (eight to ten keys fill one; of a mixed batch half the requests are
-  // taken to write), each with room for three times the average requests of a node (4 to
-  // 16), 512 MB in all at most.  What does not fit is left to batch_kernel.
+  // may be written and a quarter more (eight to ten keys fill a node; of a mixed batch half
+  // the requests are taken to write), each with room for three times the average requests
+  // of a node (4 to 16), 512 MB in all at most.  What does not fit is left to
+  // batch_kernel.
   struct group_size {
     uint64_t slots, room;
   };
@@ -1076,8 +1080,7 @@ struct gpu_masstree {
   static group_size group_shape(uint64_t n, uint64_t size, bool mixed) {
     const uint64_t writes = mixed ? n / 2 : n;
     const uint64_t nodes = std::max<uint64_t>(64, std::min<uint64_t>(writes, size / 8));
-    group_size g{64, 4};
-    while (g.slots * 20 < nodes * 23 && g.slots < kMaxGroupSlots) g.slots *= 2;
+    group_size g{std::min<uint64_t>(kMaxGroupSlots, (nodes + nodes / 4 + 63) / 64 * 64), 4};
     while (g.room < indexingpu_amd::kGroupTake && g.room * nodes < 3 * writes &&
            2 * g.room * g.slots <= kMaxGroupRooms)
       g.room *= 2;

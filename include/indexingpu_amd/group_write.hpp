@@ -37,16 +37,17 @@ namespace indexingpu_amd {
 struct group_view {
   u64* heads;
   uint4* body;
-  u32 slots;  // a power of two, at least 64
+  u32 slots;  // a multiple of 64
   u32 room;   // requests a slot holds: a power of two, at most kGroupTake
   u32* status;
   u32* claims;  // first of the bitmap words that group_write_kernel's waves begin with
   u32 waves;    // those waves (0: the launch stores no records)
-  u32 words;    // bitmap words a wave takes from the claim cursor at once
+  u32 words;    // bitmap words dealt to each of them
   u32 window;   // table slots a wave takes at once (4 .. 64)
 };
 constexpr u32 kGroupTake = 16;    // requests of one node that one tile applies
 constexpr u32 kGroupProbes = 32;  // table slots a request looks at
+constexpr u32 kWaveWords = 2;     // bitmap words of a wave's step of the claim cursor
 
 __device__ __forceinline__ u64 launch_range(const batch_args& a, u64& lo) {
   u64 hi = a.n;
@@ -60,9 +61,8 @@ __device__ __forceinline__ u64 launch_range(const batch_args& a, u64& lo) {
 
 // Adds a request to the slot of `node`, if there is room.
 __device__ __forceinline__ void group_join(const group_view& g, u32 node, const uint4& req) {
-  const u32 mask = g.slots - 1;
-  u32 h = (node * 0x9E3779B1u) >> 7 & mask;
-  for (u32 probe = 0; probe < kGroupProbes; probe++, h = (h + 1) & mask) {
+  u32 h = __umulhi(node * 0x9E3779B1u, g.slots);
+  for (u32 probe = 0; probe < kGroupProbes; probe++, h = h + 1 < g.slots ? h + 1 : 0u) {
     const u64 cur = dev::coherent_load(g.heads + h);
     u32* head = reinterpret_cast<u32*>(g.heads + h);
     u32 at = slot_lo(cur);
@@ -134,10 +134,10 @@ __global__ void __launch_bounds__(kBlockThreads) group_build_kernel(batch_args a
 }
 
 // Slabs of one wave (uniform over it): the free bits of a claimed bitmap word, and the words
-// the wave goes on with.  Every cursor step is an atomic on one address for all waves, which
-// take a good 10 ns each (4M inserts: 131K steps of one word are 1.6 ms), so a wave steps by
-// g.words words, and its first ones are dealt out by group_build_kernel: words
-// [*g.claims + wave * g.words, + g.words).
+// the wave goes on with.  A cursor step is an atomic on one address for all waves, which
+// takes a good 10 ns (4M inserts: 131K steps of one word are 1.6 ms), so most words are
+// dealt out by group_build_kernel -- words [*g.claims + wave * g.words, + g.words) -- and a
+// wave that needs more steps by kWaveWords.
 struct wave_slabs {
   u32 word = 0;
   u32 bits = 0;
@@ -164,7 +164,7 @@ __device__ __forceinline__ u32 nth_set_bit(u32 m, u32 r) {
 // The next bitmap word of the wave with free slabs (ws.word, ws.bits); false: none.  The
 // word at the wave's cursor is simply taken; once one was full, the wave looks at 64 words
 // at a time (the cursor regularly enters the part of the pool that the tree fills).
-__device__ __forceinline__ bool wave_claim(const slab_pool_view& v, wave_slabs& ws, u32 words) {
+__device__ __forceinline__ bool wave_claim(const slab_pool_view& v, wave_slabs& ws) {
   const u32 lane = threadIdx.x & 63u;
   if (v.limits) {  // linear allocator: the active region grows on misses
     u32 w = 0, b = 0;
@@ -178,7 +178,7 @@ __device__ __forceinline__ bool wave_claim(const slab_pool_view& v, wave_slabs& 
   bool look = false;
   for (u64 seen = 0; seen <= (u64)nw + 64;) {
     if (ws.left == 0) {
-      const u32 step = look ? 64u : words;
+      const u32 step = look ? 64u : kWaveWords;
       u32 c = 0;
       if (lane == 0) c = dev::atomic_add(v.cursor, step);
       ws.next = (u32)__builtin_amdgcn_readfirstlane((int)c);
@@ -208,13 +208,12 @@ __device__ __forceinline__ bool wave_claim(const slab_pool_view& v, wave_slabs& 
 
 // A slab for every lane with `need` (kInvalid where the pool has none).  Every lane of the
 // wave calls it.
-__device__ __forceinline__ u32 wave_alloc(const slab_pool_view& v, wave_slabs& ws, u32 words,
-                                          bool need) {
+__device__ __forceinline__ u32 wave_alloc(const slab_pool_view& v, wave_slabs& ws, bool need) {
   const u32 lane = threadIdx.x & 63u;
   u32 idx = kInvalid;
   u64 m = __ballot(need);
   while (m) {
-    if (ws.bits == 0 && (ws.dry || !wave_claim(v, ws, words))) {
+    if (ws.bits == 0 && (ws.dry || !wave_claim(v, ws))) {
       ws.dry = true;
       break;
     }
@@ -429,7 +428,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv
       }
       settle();
       want = (T > cap && insm) ? (root ? 2u : 1u) : 0u;
-      new_node = wave_alloc(tv.pool, ws, g.words, slot < want);
+      new_node = wave_alloc(tv.pool, ws, slot < want);
       first_new = c.bcast(new_node, 0);
       second_new = c.bcast(new_node, 1);
       if (want && (first_new == kInvalid || (want == 2 && second_new == kInvalid))) {
@@ -446,7 +445,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv
       if (store && !rec) new_val = a.values[(u64)i * maxV];
       {
         const bool one = rec && slabs == 1;
-        const u32 s0 = wave_alloc(tv.pool, ws, g.words, one);
+        const u32 s0 = wave_alloc(tv.pool, ws, one);
         if (one) new_val = s0;
         if (one && s0 == kInvalid) {
           act = aRest;
@@ -499,7 +498,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv
         const u32 r = m ? (u32)__builtin_ctz(m) : 0u;
         const u32 ii = c.bcast(i, r), tl = c.bcast(tail, r), tot = c.bcast(total, r);
         u32 count = m ? rec_num_slabs(tot) : 0u;
-        const u32 idx = wave_alloc(tv.pool, ws, g.words, slot < count);
+        const u32 idx = wave_alloc(tv.pool, ws, slot < count);
         if ((u32)__popc(c.ballot(idx != kInvalid)) < count) {  // out of slabs: left
           if (idx != kInvalid) dev::free_slab(tv.pool, idx);
           if (slot == r) act = aRest;
@@ -701,7 +700,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_link_kernel(tree_view tv,
       okm = c.ballot(ok);
       u32 T = nk + (u32)__popc(okm);
       const bool wants = okm && T > cap;
-      const u32 fresh = c.bcast(wave_alloc(tv.pool, ws, 1, wants && slot == 0), 0);
+      const u32 fresh = c.bcast(wave_alloc(tv.pool, ws, wants && slot == 0), 0);
       if (wants && fresh == kInvalid) {  // out of slabs: what fits
         if (ok && nk + (u32)__popc(okm & below_me) >= cap) ok = false;
       }

@@ -34,7 +34,16 @@ struct gmt_impl {
       alloc.reset(new alloc_t(indexingpu_amd::pool_bytes{pool_bytes}));
     else
       alloc.reset(new alloc_t(pool_ratio > 0.f ? pool_ratio : 0.9f));
-    reclaim.reset(retire_capacity ? new reclaim_t(retire_capacity) : new reclaim_t());
+    if (retire_capacity) {
+      reclaim.reset(new reclaim_t(retire_capacity));
+    } else {
+      // A launch retires a slab once at most, so the default list (2^26 entries, 256 MB)
+      // need not be longer than the pool and the entries that pad tiles' reservations.
+      // Allocating and freeing it is part of every index a program makes: freeing device
+      // memory takes up to 25 us a MB here.
+      const uint64_t most = alloc->total_slabs() + (1ull << 20);
+      reclaim.reset(most < (1ull << 26) ? new reclaim_t((uint32_t)most) : new reclaim_t());
+    }
     t16.reset(new tree_t<16>(*alloc, *reclaim));
     t32.reset(new tree_t<32>(*t16));
     t64.reset(new tree_t<64>(*t16));
