@@ -209,6 +209,11 @@ int gmt_set_mixed_split(gmt_index* index, uint32_t min_requests);
  * not depend on it. */
 int gmt_set_write_hints(gmt_index* index, uint32_t min_requests);
 
+/* Closed indexes leave device memory (at most 1/32 of the device's) for the next ones, since
+ * the driver's wipe of freed memory is slower than a bulk load; a block not taken again soon,
+ * or when an allocation of the library fails, is freed.  This frees all of it now. */
+int gmt_release_memory(void);
+
 /* Hinted write batches of at least min_requests requests (default 8192), and split mixed
  * batches of at least twice as many, apply their writes border node by border node before
  * the step machine runs what is left; 0xFFFFFFFF turns this off.  Uses scratch beside the

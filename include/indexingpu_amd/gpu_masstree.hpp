@@ -18,6 +18,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "block_cache.hpp"
 #include "device_context.hpp"
 #include "group_write.hpp"
 #include "hip_util.hpp"
@@ -125,13 +126,13 @@ struct gpu_masstree {
         shortcut_on_(false) {}
   gpu_masstree& operator=(const gpu_masstree&) = delete;
   ~gpu_masstree() {
-    if (scan_stack_) (void)hipFree(scan_stack_);  // per instance, never shared
-    if (park_) (void)hipFree(park_);
-    if (hints_) (void)hipFree(hints_);
-    if (group_heads_) (void)hipFree(group_heads_);
-    if (group_body_) (void)hipFree(group_body_);
-    if (group_status_) (void)hipFree(group_status_);
-    if (shortcut_) (void)hipFree(shortcut_);
+    indexingpu_amd::device_give(scan_stack_);  // per instance, never shared
+    indexingpu_amd::device_give(park_);
+    indexingpu_amd::device_give(hints_);
+    indexingpu_amd::device_give(group_heads_);
+    indexingpu_amd::device_give(group_body_);
+    indexingpu_amd::device_give(group_status_);
+    indexingpu_amd::device_give(shortcut_);
     if (owner_) {
       if (err_) (void)hipFree(err_);
       if (barrier_) (void)hipFree(barrier_);
@@ -411,7 +412,7 @@ struct gpu_masstree {
     shortcut_on_ = on && owner_;
     if (!on && shortcut_) {
       IGPU_HIP_TRY(hipDeviceSynchronize());
-      IGPU_HIP_TRY(hipFree(shortcut_));
+      indexingpu_amd::device_give(shortcut_);
       shortcut_ = nullptr;
       shortcut_bits_ = shortcut_capacity_bits_ = 0;
       shortcut_size_ = 0;
@@ -838,9 +839,10 @@ struct gpu_masstree {
     if (bits > shortcut_capacity_bits_) {
       // level-1 table, border-level table (2^capacity entries each), built-at merge count
       IGPU_HIP_TRY(hipDeviceSynchronize());
-      if (shortcut_) IGPU_HIP_TRY(hipFree(shortcut_));
+      indexingpu_amd::device_give(shortcut_);
       shortcut_ = nullptr;
-      IGPU_HIP_TRY(hipMalloc(&shortcut_, (8ull << bits) + 256));
+      shortcut_bits_ = shortcut_capacity_bits_ = 0;
+      IGPU_HIP_TRY(indexingpu_amd::device_take(&shortcut_, (8ull << bits) + 256));
       shortcut_capacity_bits_ = bits;
     }
     const uint32_t entries = 1u << bits;
@@ -931,7 +933,7 @@ struct gpu_masstree {
     const uint64_t n = a.n;
     if (n == 0) return;
     auto room = [&]() {
-      const bool grouped = write_group_min_ != 0xFFFFFFFFu && size >= write_group_min_;
+      const bool grouped = groups_on() && size >= write_group_min_;
       return std::max<uint64_t>(kGrowthMin,
                                 grouped ? size / kGrowthGrouped : size * (kGrowthFactor - 1));
     };
@@ -946,7 +948,7 @@ struct gpu_masstree {
     const uint64_t chunk = std::min<uint64_t>(n, kHintChunk);
     if (write_hint_min_ != 0xFFFFFFFFu && n >= write_hint_min_) {
       ensure_hints(chunk);
-      if (write_group_min_ != 0xFFFFFFFFu && n >= write_group_min_)
+      if (groups_on() && n >= write_group_min_)
         ensure_groups(chunk, group_shape(chunk, (size + n) / 3 * 2, false), stream);
     }
     uint64_t done = 0;
@@ -1017,17 +1019,17 @@ struct gpu_masstree {
   static constexpr uint64_t kMaxGroupSlots = 1ull << 23;
   static constexpr uint64_t kLinkShare = 4;
   static constexpr uint64_t kMaxDealtWords = 32;
+  // Trees whose nodes split below the layout's maximum (set_fanout) are written by the step
+  // machine: groups fill nodes differently.
+  bool groups_on() const { return write_group_min_ != 0xFFFFFFFFu && fanout_flags_ == 0; }
   // `added`: keys that earlier launches of the batch may have inserted.
   void launch_groups(indexingpu_amd::batch_args& a, uint64_t n, hipStream_t stream,
                      uint64_t added = 0) {
     // of a mixed batch half the requests are taken to write
-    if (write_group_min_ == 0xFFFFFFFFu || (a.types ? n / 2 : n) < write_group_min_ ||
-        n >= (1ull << 31))
-      return;
+    if (!groups_on() || (a.types ? n / 2 : n) < write_group_min_ || n >= (1ull << 31)) return;
     const uint64_t size = *inserted_hint_ + added;
     const group_size shape = group_shape(n, size, a.types != nullptr);
     if (!ensure_groups(n, shape, stream)) return;
-    a.flags |= fanout_flags_;
     const uint32_t threads = indexingpu_amd::kBlockThreads;
     auto build = indexingpu_amd::group_build_kernel;
     const auto grid = [&](uint64_t work, auto kernel) {
@@ -1097,10 +1099,10 @@ struct gpu_masstree {
     IGPU_HIP_TRY(hipDeviceSynchronize());
     auto grow = [](auto*& ptr, uint64_t& have, uint64_t want, uint64_t bytes) {
       if (want <= have) return true;
-      if (ptr) IGPU_HIP_TRY(hipFree(ptr));
+      indexingpu_amd::device_give(ptr);
       ptr = nullptr;
       have = 0;
-      if (hipMalloc(&ptr, want * bytes + 128) != hipSuccess) {
+      if (indexingpu_amd::device_take(&ptr, want * bytes + 128) != hipSuccess) {
         (void)hipGetLastError();
         ptr = nullptr;
         return false;
@@ -1253,24 +1255,30 @@ struct gpu_masstree {
   void ensure_park(uint64_t n) {
     if (n <= park_words_) return;
     IGPU_HIP_TRY(hipDeviceSynchronize());
-    if (park_) IGPU_HIP_TRY(hipFree(park_));
-    IGPU_HIP_TRY(hipMalloc(&park_, n * 4));
+    indexingpu_amd::device_give(park_);
+    park_ = nullptr;
+    park_words_ = 0;
+    IGPU_HIP_TRY(indexingpu_amd::device_take(&park_, n * 4));
     park_words_ = n;
   }
   // start hints of the writes of split mixed batches (kHintWords words per request)
   void ensure_hints(uint64_t n) {
     if (n <= hint_requests_) return;
     IGPU_HIP_TRY(hipDeviceSynchronize());
-    if (hints_) IGPU_HIP_TRY(hipFree(hints_));
-    IGPU_HIP_TRY(hipMalloc(&hints_, n * 4 * indexingpu_amd::kHintWords));
+    indexingpu_amd::device_give(hints_);
+    hints_ = nullptr;
+    hint_requests_ = 0;
+    IGPU_HIP_TRY(indexingpu_amd::device_take(&hints_, n * 4 * indexingpu_amd::kHintWords));
     hint_requests_ = n;
   }
 
   void ensure_scan_stack(uint64_t words) {
     if (words <= scan_stack_words_) return;
     IGPU_HIP_TRY(hipDeviceSynchronize());
-    if (scan_stack_) IGPU_HIP_TRY(hipFree(scan_stack_));
-    IGPU_HIP_TRY(hipMalloc(&scan_stack_, words * 4));
+    indexingpu_amd::device_give(scan_stack_);
+    scan_stack_ = nullptr;
+    scan_stack_words_ = 0;
+    IGPU_HIP_TRY(indexingpu_amd::device_take(&scan_stack_, words * 4));
     scan_stack_words_ = words;
   }
 

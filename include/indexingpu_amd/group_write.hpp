@@ -284,8 +284,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv
   launch_range(a, lo);
   const u32 num_slabs = tv.pool.num_slabs;
   const u32 maxK = a.max_key_length, maxV = a.max_value_length;
-  const u32 cap_bits = (a.flags >> kReqBorderCapShift) & 15u;
-  const u32 cap = cap_bits ? cap_bits : kBorderCap;
+  constexpr u32 cap = kBorderCap;
   const u32 step = gridDim.x * (kBlockThreads / 64) * g.window;
   // after a corruption or livelock guard fired batch_kernel skips the requests
   const u32 err = *tv.err;
@@ -632,8 +631,7 @@ __global__ void __launch_bounds__(kBlockThreads) group_link_kernel(tree_view tv,
   const wave_tile<16, true> c(tv.pool, tv.retire, tv.err, tv.root);
   const u32 lane64 = threadIdx.x & 63u, slot = c.slot, tile = lane64 >> 4;
   const u32 below_me = (1u << slot) - 1u;
-  const u32 cap_bits = (a.flags >> kReqInteriorCapShift) & 15u;
-  const u32 cap = cap_bits ? cap_bits : kInteriorCap;
+  constexpr u32 cap = kInteriorCap;
   const u32 version_mask = ~((1u << kVersionShift) - 1u);
   __shared__ u64 items[kBlockThreads / 16][32];  // a tile's (low bound, child), in order
   u64* const it = items[threadIdx.x / 16];

@@ -26,6 +26,7 @@
 #pragma once
 #include <cstdint>
 
+#include "block_cache.hpp"
 #include "hip_util.hpp"
 #include "layout.hpp"
 
@@ -73,10 +74,10 @@ class simple_debra_reclaimer {
   }
   explicit simple_debra_reclaimer(uint32_t capacity_entries) { init(capacity_entries); }
   ~simple_debra_reclaimer() {
-    if (view_.list) (void)hipFree(view_.list);
+    device_give(view_.list);
     if (view_.count) (void)hipFree(view_.count);
-    if (view_.announce) (void)hipFree(view_.announce);
-    if (view_.bags) (void)hipFree(view_.bags);
+    device_give(view_.announce);
+    device_give(view_.bags);
   }
   simple_debra_reclaimer(const simple_debra_reclaimer&) = delete;
   simple_debra_reclaimer& operator=(const simple_debra_reclaimer&) = delete;
@@ -100,7 +101,7 @@ class simple_debra_reclaimer {
   void init(u32 cap) {
     view_.capacity = cap;
     view_.enabled = 1;
-    IGPU_HIP_TRY(hipMalloc(&view_.list, sizeof(u32) * (size_t)cap));
+    IGPU_HIP_TRY(device_take(&view_.list, sizeof(u32) * (size_t)cap));
     IGPU_HIP_TRY(hipMalloc(&view_.count, 256));
     IGPU_HIP_TRY(hipMemset(view_.count, 0, 256));
     view_.leaked = view_.count + 1;
@@ -108,10 +109,10 @@ class simple_debra_reclaimer {
     // device-API epochs: announce entries for up to kMaxBlocks blocks per launch and
     // buffer_size_per_block bytes of limbo bags for each of up to kBagBlocks blocks
     view_.max_blocks = kMaxBlocks;
-    IGPU_HIP_TRY(hipMalloc(&view_.announce, 4ull * kMaxBlocks));
+    IGPU_HIP_TRY(device_take(&view_.announce, 4ull * kMaxBlocks));
     IGPU_HIP_TRY(hipMemset(view_.announce, 0, 4ull * kMaxBlocks));
     view_.bag_words = (u32)((uint64_t)buffer_size_per_block / 4 * kBagBlocks);
-    IGPU_HIP_TRY(hipMalloc(&view_.bags, 4ull * view_.bag_words));
+    IGPU_HIP_TRY(device_take(&view_.bags, 4ull * view_.bag_words));
     IGPU_HIP_TRY(hipMemset(view_.bags, 0, 4ull * view_.bag_words));
     IGPU_HIP_TRY(hipDeviceSynchronize());
   }

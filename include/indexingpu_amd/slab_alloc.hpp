@@ -19,6 +19,7 @@
 #include <utility>
 #include <vector>
 
+#include "block_cache.hpp"
 #include "hip_util.hpp"
 #include "layout.hpp"
 
@@ -68,7 +69,7 @@ class simple_slab_allocator {
   }
   explicit simple_slab_allocator(pool_bytes b) { init(b.bytes); }
   ~simple_slab_allocator() {
-    if (base_) (void)hipFree(base_);
+    device_give(base_);
   }
   simple_slab_allocator(const simple_slab_allocator&) = delete;
   simple_slab_allocator& operator=(const simple_slab_allocator&) = delete;
@@ -97,7 +98,7 @@ class simple_slab_allocator {
     std::size_t bitmap_bytes = (std::size_t)view_.num_words * 4;
     std::size_t head = (bitmap_bytes + 256 + 255) / 256 * 256;  // bitmap + cursor, aligned
     std::size_t total = head + (std::size_t)slabs * kSlabBytes;
-    IGPU_HIP_TRY(hipMalloc(&base_, total));
+    IGPU_HIP_TRY(device_take(&base_, total));
     IGPU_HIP_TRY(hipMemset(base_, 0, head));
     view_.bitmap = reinterpret_cast<u32*>(base_);
     view_.cursor = reinterpret_cast<u32*>(reinterpret_cast<char*>(base_) + bitmap_bytes);
@@ -136,7 +137,7 @@ class simple_slab_linear_allocator {
     init(b.bytes, initial_slab_ratio);
   }
   ~simple_slab_linear_allocator() {
-    if (base_) (void)hipFree(base_);
+    device_give(base_);
   }
   simple_slab_linear_allocator(const simple_slab_linear_allocator&) = delete;
   simple_slab_linear_allocator& operator=(const simple_slab_linear_allocator&) = delete;
@@ -175,7 +176,7 @@ class simple_slab_linear_allocator {
     std::size_t bitmap_bytes = (std::size_t)view_.num_words * 4;
     std::size_t head = (bitmap_bytes + 512 + 255) / 256 * 256;  // bitmap, cursor, limits
     std::size_t total = head + (std::size_t)slabs * kSlabBytes;
-    IGPU_HIP_TRY(hipMalloc(&base_, total));
+    IGPU_HIP_TRY(device_take(&base_, total));
     IGPU_HIP_TRY(hipMemset(base_, 0, head));
     view_.bitmap = reinterpret_cast<u32*>(base_);
     view_.cursor = reinterpret_cast<u32*>(reinterpret_cast<char*>(base_) + bitmap_bytes);

@@ -418,6 +418,10 @@ int gmt_set_write_hints(gmt_index* index, uint32_t min_requests) {
   return GMT_OK;
 }
 
+int gmt_release_memory(void) {
+  return guarded([] { indexingpu_amd::release_kept(); });
+}
+
 int gmt_set_write_groups(gmt_index* index, uint32_t min_requests) {
   if (!index) return bad("gmt_set_write_groups: null handle");
   B(index)->on_all([&](auto& t) { t.set_write_groups(min_requests); });

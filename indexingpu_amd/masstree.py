@@ -95,6 +95,12 @@ def load_library():
     return lib
 
 
+def release_memory():
+    """Frees the device memory that closed indexes left for the next ones."""
+    if load_library().gmt_release_memory() != 0:
+        raise MasstreeError(load_library().gmt_last_error_message().decode())
+
+
 def _ptr(t, esize, name, need=0):
     """Device pointer of a contiguous CUDA tensor with elements of `esize` bytes and at
     least `need` elements (checked here, so a kernel never indexes past a buffer)."""
