@@ -894,8 +894,8 @@ struct gpu_masstree {
   // launches).  The batch therefore runs as consecutive launches that each grow the
   // tree at most kGrowthFactor-fold (from kGrowthMin keys; by kGrowthGrouped once their
   // writes are grouped), then the rest in one launch.
-  // The launches take the requests in a scattered order (index times a multiplier coprime to n, modulo n), so
-  // each one is a sample of the whole batch: a batch in key order -- or one whose keys
+  // The launches take the requests in a scattered order (index times a multiplier coprime
+  // to n, modulo n), so each one is a sample of the whole batch: a batch in key order -- or one whose keys
   // all lie past the tree's current right edge -- then grows every key range at once
   // instead of sending every tile to the same edge node.  The requests of one batch are
   // independent, so any order gives the results of one launch.  The size estimate

@@ -419,102 +419,104 @@ __global__ void __launch_bounds__(kBlockThreads) group_write_kernel(tree_view tv
       u32 want = 0, new_node = kInvalid, first_new = kInvalid, second_new = kInvalid;  // new nodes
       u32 new_ks = kValue, new_val = kInvalid;  // what an inserted or replaced entry holds
       if constexpr (Stores) {
-      // at most two nodes: equal slices stay together, so up to 2 cap - 1 entries
-      {
-        const u32 ns = (u32)__popc(survm);
-        const u32 room = 2 * cap - 1 > ns ? 2 * cap - 1 - ns : 0u;
-        if (T > cap && act == aInsert && (u32)__popc(insm & below_me) >= room) act = aRest;
-      }
-      settle();
-      want = (T > cap && insm) ? (root ? 2u : 1u) : 0u;
-      new_node = wave_alloc(tv.pool, ws, slot < want);
-      first_new = c.bcast(new_node, 0);
-      second_new = c.bcast(new_node, 1);
-      if (want && (first_new == kInvalid || (want == 2 && second_new == kInvalid))) {
-        if (new_node != kInvalid) dev::free_slab(tv.pool, new_node);
-        if (act == aInsert) act = aRest;
-        want = 0;
-      }
-      // ---- records of inserted and replaced values
-      const bool store = act == aInsert || act == aReplace;
-      new_ks = more ? kSuffix : (vlen == 1 ? kValue : kLongVal);
-      const u32 total = 1 + tail + vlen;
-      const u32 slabs = rec_num_slabs(total);
-      bool rec = store && new_ks != kValue;
-      if (store && !rec) new_val = a.values[(u64)i * maxV];
-      {
-        const bool one = rec && slabs == 1;
-        const u32 s0 = wave_alloc(tv.pool, ws, one);
-        if (one) new_val = s0;
-        if (one && s0 == kInvalid) {
-          act = aRest;
-          rec = false;
+        // at most two nodes: equal slices stay together, so up to 2 cap - 1 entries
+        {
+          const u32 ns = (u32)__popc(survm);
+          const u32 room = 2 * cap - 1 > ns ? 2 * cap - 1 - ns : 0u;
+          if (T > cap && act == aInsert && (u32)__popc(insm & below_me) >= room) act = aRest;
         }
-      }
-      auto word = [&](u32 ii, u32 ll, u32 tl, u32 tot, u32 d) -> u32 {
-        if (d == 0) return rec_len_word(tl, tot - 1 - tl);
-        if (d >= tot) return 0;
-        return d <= tl ? a.keys[(u64)ii * maxK + ll + d] : a.values[(u64)ii * maxV + (d - 1 - tl)];
-      };
-      // Records of one slab are stored in halves of 64 bytes (the second only where it is
-      // filled), eight lanes and one coalesced store each: the halves of the wave's four
-      // groups are listed in LDS, so the wave takes eight at a time whoever they belong to.
-      {
-        const bool one = rec && slabs == 1, two = one && total > 16;
-        const u64 m1 = __ballot(one), m2 = __ballot(two);
-        const u64 lt = (1ull << lane64) - 1ull;
-        const u32 n1 = (u32)__popcll(m1), halves = n1 + (u32)__popcll(m2);
-        if (one) half_of[wave_in_block][__popcll(m1 & lt)] = (uint8_t)lane64;
-        if (two) half_of[wave_in_block][n1 + __popcll(m2 & lt)] = (uint8_t)(lane64 | 64u);
-        lds_order();
-        for (u32 s0 = 0; s0 < halves; s0 += 16) {
-          u32 x0[2], x1[2], at[2], dd[2];
-#pragma unroll
-          for (u32 j = 0; j < 2; j++) {
-            const u32 s = s0 + 8 * j + (lane64 >> 3);
-            const u32 e = s < halves ? half_of[wave_in_block][s] : 0u;
-            const int r = (int)(e & 63u);
-            const u32 ii = __shfl(i, r, 64), ll = __shfl(l, r, 64), rz = __shfl(req.z, r, 64);
-            const u32 tl = rz & 0xFFFFu, tot = 1 + tl + (rz >> 16);
-            const u32 d = (e >> 6) * 16 + 2 * (lane64 & 7u);
-            at[j] = __shfl(new_val, r, 64);
-            dd[j] = d / 2;
-            x0[j] = x1[j] = 0;
-            if (s < halves) {
-              x0[j] = word(ii, ll, tl, tot, d);
-              x1[j] = d + 1 == kRecordNextWord ? kInvalid : word(ii, ll, tl, tot, d + 1);
-            }
+        settle();
+        want = (T > cap && insm) ? (root ? 2u : 1u) : 0u;
+        new_node = wave_alloc(tv.pool, ws, slot < want);
+        first_new = c.bcast(new_node, 0);
+        second_new = c.bcast(new_node, 1);
+        if (want && (first_new == kInvalid || (want == 2 && second_new == kInvalid))) {
+          if (new_node != kInvalid) dev::free_slab(tv.pool, new_node);
+          if (act == aInsert) act = aRest;
+          want = 0;
+        }
+        // ---- records of inserted and replaced values
+        const bool store = act == aInsert || act == aReplace;
+        new_ks = more ? kSuffix : (vlen == 1 ? kValue : kLongVal);
+        const u32 total = 1 + tail + vlen;
+        const u32 slabs = rec_num_slabs(total);
+        bool rec = store && new_ks != kValue;
+        if (store && !rec) new_val = a.values[(u64)i * maxV];
+        {
+          const bool one = rec && slabs == 1;
+          const u32 s0 = wave_alloc(tv.pool, ws, one);
+          if (one) new_val = s0;
+          if (one && s0 == kInvalid) {
+            act = aRest;
+            rec = false;
           }
+        }
+        auto word = [&](u32 ii, u32 ll, u32 tl, u32 tot, u32 d) -> u32 {
+          if (d == 0) return rec_len_word(tl, tot - 1 - tl);
+          if (d >= tot) return 0;
+          return d <= tl ? a.keys[(u64)ii * maxK + ll + d]
+                         : a.values[(u64)ii * maxV + (d - 1 - tl)];
+        };
+        // Records of one slab are stored in halves of 64 bytes (the second only where it is
+        // filled), eight lanes and one coalesced store each: the halves of the wave's four
+        // groups are listed in LDS, so the wave takes eight at a time whoever they belong to.
+        {
+          const bool one = rec && slabs == 1, two = one && total > 16;
+          const u64 m1 = __ballot(one), m2 = __ballot(two);
+          const u64 lt = (1ull << lane64) - 1ull;
+          const u32 n1 = (u32)__popcll(m1), halves = n1 + (u32)__popcll(m2);
+          if (one) half_of[wave_in_block][__popcll(m1 & lt)] = (uint8_t)lane64;
+          if (two) half_of[wave_in_block][n1 + __popcll(m2 & lt)] = (uint8_t)(lane64 | 64u);
+          lds_order();
+          for (u32 s0 = 0; s0 < halves; s0 += 16) {
+            u32 x0[2], x1[2], at[2], dd[2];
 #pragma unroll
-          for (u32 j = 0; j < 2; j++)
-            if (s0 + 8 * j + (lane64 >> 3) < halves)
-              dev::coherent_store(c.slab(at[j]) + dd[j], slot_make(x0[j], x1[j]));
+            for (u32 j = 0; j < 2; j++) {
+              const u32 s = s0 + 8 * j + (lane64 >> 3);
+              const u32 e = s < halves ? half_of[wave_in_block][s] : 0u;
+              const int r = (int)(e & 63u);
+              const u32 ii = __shfl(i, r, 64), ll = __shfl(l, r, 64), rz = __shfl(req.z, r, 64);
+              const u32 tl = rz & 0xFFFFu, tot = 1 + tl + (rz >> 16);
+              const u32 d = (e >> 6) * 16 + 2 * (lane64 & 7u);
+              at[j] = __shfl(new_val, r, 64);
+              dd[j] = d / 2;
+              x0[j] = x1[j] = 0;
+              if (s < halves) {
+                x0[j] = word(ii, ll, tl, tot, d);
+                x1[j] = d + 1 == kRecordNextWord ? kInvalid : word(ii, ll, tl, tot, d + 1);
+              }
+            }
+#pragma unroll
+            for (u32 j = 0; j < 2; j++)
+              if (s0 + 8 * j + (lane64 >> 3) < halves)
+                dev::coherent_store(c.slab(at[j]) + dd[j], slot_make(x0[j], x1[j]));
+          }
         }
-      }
-      // Longer records, one of each tile at a time: their slabs are neighbours where the
-      // bitmap word has that many free, one whole-line store each.
-      for (u32 m = c.ballot(rec && slabs > 1); __ballot(m != 0); m &= m - 1) {
-        const u32 r = m ? (u32)__builtin_ctz(m) : 0u;
-        const u32 ii = c.bcast(i, r), tl = c.bcast(tail, r), tot = c.bcast(total, r);
-        u32 count = m ? rec_num_slabs(tot) : 0u;
-        const u32 idx = wave_alloc(tv.pool, ws, slot < count);
-        if ((u32)__popc(c.ballot(idx != kInvalid)) < count) {  // out of slabs: left
-          if (idx != kInvalid) dev::free_slab(tv.pool, idx);
-          if (slot == r) act = aRest;
-          count = 0;
+        // Longer records, one of each tile at a time: their slabs are neighbours where the
+        // bitmap word has that many free, one whole-line store each.
+        for (u32 m = c.ballot(rec && slabs > 1); __ballot(m != 0); m &= m - 1) {
+          const u32 r = m ? (u32)__builtin_ctz(m) : 0u;
+          const u32 ii = c.bcast(i, r), tl = c.bcast(tail, r), tot = c.bcast(total, r);
+          u32 count = m ? rec_num_slabs(tot) : 0u;
+          const u32 idx = wave_alloc(tv.pool, ws, slot < count);
+          if ((u32)__popc(c.ballot(idx != kInvalid)) < count) {  // out of slabs: left
+            if (idx != kInvalid) dev::free_slab(tv.pool, idx);
+            if (slot == r) act = aRest;
+            count = 0;
+          }
+          const u32 head = c.bcast(idx, 0);
+          if (count && slot == r) new_val = head;
+          for (u32 s = 0; __ballot(s < count); s++) {
+            const u32 at = c.bcast(idx, s & 15u), nxt = c.bcast(idx, (s + 1) & 15u);
+            if (s >= count) continue;
+            const u32 d = s * kRecordWordsPerSlab + 2 * slot;
+            const u32 x0 = word(ii, l, tl, tot, d);
+            const u32 x1 =
+                slot < 15 ? word(ii, l, tl, tot, d + 1) : (s + 1 < count ? nxt : kInvalid);
+            dev::coherent_store(c.slab(at) + slot, slot_make(x0, x1));
+          }
         }
-        const u32 head = c.bcast(idx, 0);
-        if (count && slot == r) new_val = head;
-        for (u32 s = 0; __ballot(s < count); s++) {
-          const u32 at = c.bcast(idx, s & 15u), nxt = c.bcast(idx, (s + 1) & 15u);
-          if (s >= count) continue;
-          const u32 d = s * kRecordWordsPerSlab + 2 * slot;
-          const u32 x0 = word(ii, l, tl, tot, d);
-          const u32 x1 = slot < 15 ? word(ii, l, tl, tot, d + 1) : (s + 1 < count ? nxt : kInvalid);
-          dev::coherent_store(c.slab(at) + slot, slot_make(x0, x1));
-        }
-      }
-      settle();
+        settle();
       }
       // the erase that would empty the node merges it away or unlinks its layer: left
       {
