@@ -21,9 +21,10 @@
 // see what they see of the step machine: the header is locked before the first store to a
 // node, every store is coherent and complete before the unlocked header is stored.
 //
-// Measured on MI355X (16M keys of 2..8 slices, 2-slice values), the launches that write: 4M
-// inserts 5.0 -> 1.5 ms, 4M erases 3.4 -> 1.0 ms, 1M updates of 8-slice values on 4M keys
-// 1.03 -> 0.46 ms, the 105K writes of a 1M mixed batch on 64M keys 0.27 -> 0.11 ms.
+// Measured on MI355X (16M keys of 2..8 slices, 2-slice values), the launches that write, step
+// machine -> group_write_kernel: 4M inserts 5.0 -> 0.9 ms, 4M erases 3.4 -> 0.5 ms, 1M updates
+// of 8-slice values on 4M keys 1.03 -> 0.26 ms, the 105K writes of a 1M mixed batch on 64M keys
+// 0.27 -> 0.06 ms.  The group build takes 0.4, 0.4, 0.11 and 0.02 ms of that back.
 #pragma once
 #include "kernels.hpp"
 
